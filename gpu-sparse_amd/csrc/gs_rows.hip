@@ -15,37 +15,55 @@ __global__ void k_fill(T *p, int64_t n, T v) {
 
 // ---------------------------------------------------------------------- compacted top-k
 
-// Candidates v >= tau[b] of a [B, L] fp32 matrix: one atomic slot reservation
-// per 64 entries (wave ballot), as _compact_above_threshold_kernel does per block.
+// Candidates v >= tau[b] of a [B, L] fp32 matrix, as _compact_above_threshold_kernel
+// lists them per block.  A workgroup takes 4096 entries of a row, 16 per thread
+// loaded together, counts its candidates with wave ballots and reserves their
+// slots with one atomic: the row's counter is one address, and an atomic per 64
+// entries queued up behind it (compaction and selection of 64 rows of
+// 131072, 2% kept, k = 1000: 1005 us with one per 64 entries, 49 us with one per 4096).
+constexpr int kCompactPer = 16;  // entries per thread
 __global__ void __launch_bounds__(256)
     k_compact(const float *__restrict__ scores, int64_t ld, int64_t L, const float *__restrict__ tau,
               int32_t *__restrict__ cidx, float *__restrict__ cval, int32_t *__restrict__ counts,
               int32_t max_cand) {
+    __shared__ int32_t s_cnt[4], s_base;
     const int b = blockIdx.y;
     const float t = tau[b];
-    const int lane = gs_lane();
+    const int wave = gs_uniform((int)(threadIdx.x >> 6));
     const float *row = scores + (int64_t)b * ld;
-    for (int64_t i0 = (blockIdx.x * (int64_t)blockDim.x + (threadIdx.x & ~63)); i0 < L;
-         i0 += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t i = i0 + lane;
-        float v = 0.0f;
-        bool keep = false;
-        if (i < L) {
-            v = row[i];
-            keep = v >= t;
-        }
-        const uint64_t m = __ballot(keep);
-        if (m == 0) continue;
-        int32_t base = 0;
-        if (lane == 0) base = atomicAdd(counts + b, (int32_t)__popcll(m));
-        base = __shfl(base, 0, 64);
-        if (keep) {
-            const int32_t slot = base + (int32_t)__popcll(m & gs_lanemask_lt());
+    const int64_t i0 = blockIdx.x * (int64_t)(256 * kCompactPer) + threadIdx.x;
+    float v[kCompactPer];
+    uint64_t m[kCompactPer];
+#pragma unroll
+    for (int u = 0; u < kCompactPer; ++u) {
+        const int64_t i = i0 + u * 256;
+        v[u] = i < L ? row[i] : 0.0f;
+    }
+    int32_t n = 0;
+#pragma unroll
+    for (int u = 0; u < kCompactPer; ++u) {
+        m[u] = __ballot(i0 + u * 256 < L && v[u] >= t);
+        n += (int32_t)__popcll(m[u]);
+    }
+    if (gs_lane() == 0) s_cnt[wave] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int32_t tot = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+        s_base = tot ? atomicAdd(counts + b, tot) : 0;
+    }
+    __syncthreads();
+    int32_t at = s_base;
+    for (int w = 0; w < wave; ++w) at += s_cnt[w];
+#pragma unroll
+    for (int u = 0; u < kCompactPer; ++u) {
+        if (m[u] >> gs_lane() & 1ull) {
+            const int32_t slot = at + (int32_t)__popcll(m[u] & gs_lanemask_lt());
             if (slot < max_cand) {
-                cidx[(int64_t)b * max_cand + slot] = (int32_t)i;
-                cval[(int64_t)b * max_cand + slot] = v;
+                cidx[(int64_t)b * max_cand + slot] = (int32_t)(i0 + u * 256);
+                cval[(int64_t)b * max_cand + slot] = v[u];
             }
         }
+        at += (int32_t)__popcll(m[u]);
     }
 }
 
@@ -60,21 +78,21 @@ __global__ void __launch_bounds__(kSelThreads)
     const int32_t cnt = counts ? counts[b] : (int32_t)0x7FFFFFFF;
     if (tau && cnt <= max_cand) {
         SrcCandF32 src{cval + (int64_t)b * max_cand, cidx + (int64_t)b * max_cand, (int64_t)cnt};
-        const int c = block_topk<32>(src, k, sh, false);
+        const int c = block_topk<uint32_t>(src, k, sh, false);
         for (int i = threadIdx.x; i < k; i += blockDim.x) {
             const bool ok = i < c;
-            out_v[(int64_t)b * k + i] = ok ? gs_unkey_f32((uint32_t)sh.key[i]) : -INFINITY;
-            out_i[(int64_t)b * k + i] = ok ? (int64_t)sh.doc[i] : 0;
+            out_v[(int64_t)b * k + i] = ok ? gs_unkey_f32((uint32_t)sh.key_at(i)) : -INFINITY;
+            out_i[(int64_t)b * k + i] = ok ? (int64_t)sh.doc_at(i) : 0;
         }
     } else {
         // overflowed (or unthresholded) row: select from the full row, keys shifted by
         // one so that 0 marks entries below tau
         SrcRowF32 src{scores + (int64_t)b * ld, L, tau ? gs_key_f32(tau[b]) : 0u};
-        const int c = block_topk<40>(src, k, sh, true);
+        const int c = block_topk<uint64_t>(src, k, sh, true);
         for (int i = threadIdx.x; i < k; i += blockDim.x) {
             const bool ok = i < c;
-            out_v[(int64_t)b * k + i] = ok ? gs_unkey_f32((uint32_t)(sh.key[i] - 1)) : -INFINITY;
-            out_i[(int64_t)b * k + i] = ok ? (int64_t)sh.doc[i] : 0;
+            out_v[(int64_t)b * k + i] = ok ? gs_unkey_f32((uint32_t)(sh.key_at(i) - 1)) : -INFINITY;
+            out_i[(int64_t)b * k + i] = ok ? (int64_t)sh.doc_at(i) : 0;
         }
     }
 }
@@ -146,7 +164,7 @@ extern "C" int gs_compacted_topk(const float *scores_d, int64_t ld, int32_t B, i
     }
     k_fill<int32_t><<<gs_blocks(B, 256), 256, 0, s>>>(counts_d, B, 0);
     if (tau_d) {
-        dim3 g(gs_blocks(L, 256, 4096), (unsigned)B);
+        dim3 g(gs_blocks(L, 256 * kCompactPer), (unsigned)B);
         k_compact<<<g, 256, 0, s>>>(scores_d, ld, L, tau_d, cidx, cval, counts_d, max_cand);
     } else {
         k_fill<int32_t><<<gs_blocks(B, 256), 256, 0, s>>>(counts_d, B, (int32_t)L);

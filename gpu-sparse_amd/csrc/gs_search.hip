@@ -58,6 +58,7 @@ constexpr int64_t kSeedFillWgs = 256;       // workgroups (tiles x query groups)
 constexpr int64_t kSeedMaxTiles = 64;       // most tiles of a default seed widened towards that
 constexpr int64_t kPairMinWgs = 12288;    // workgroups (~48 per CU) needed before a workgroup scores two tiles
 constexpr int64_t kTripleMinWgs = 49152;  // and before it scores three
+constexpr int kCus = 256;  // compute units of the GPU
 constexpr size_t kTileLds = 144 * 1024;  // LDS of the fp64 / uint32 row tiles of one dense-path workgroup
 // LDS of the score slices of one fused-scoring workgroup (2 queries x 8192 docs):
 // two such workgroups share a CU, so one's set-up and emission (latency-bound)
@@ -1604,11 +1605,12 @@ __global__ void __launch_bounds__(256)
 // ---------------------------------------------------------------------- selection
 
 // uint8 rows: the exact top-k of the candidates is the answer.  Float rows: the
-// fixed-point k-th score tau' gives the rescoring set {fixed >= tau' - mfix}.
+// fixed-point k-th score tau' gives the rescoring set {fixed >= tau' - mfix};
+// nothing is sorted, and the first `held` keys stay in dynamic LDS over the passes.
 template <int WT>
-__global__ void __launch_bounds__(kSelThreads)
+__global__ void __launch_bounds__(kSelThreads, WT == GS_W_U8 ? 4 : 8)
     k_select_cands(const uint32_t *__restrict__ cand_doc, const uint32_t *__restrict__ cand_key,
-                   const uint32_t *__restrict__ cnt, int32_t cap, int32_t k, const uint32_t *__restrict__ mfix,
+                   const uint32_t *__restrict__ cnt, int32_t cap, int32_t k, int32_t held, const uint32_t *__restrict__ mfix,
                    uint32_t *__restrict__ resc_doc, uint32_t *__restrict__ resc_cnt, int32_t resc_cap,
                    const int32_t *__restrict__ perm, void *__restrict__ out_scores, int64_t *__restrict__ out_ids,
                    int32_t *__restrict__ status) {
@@ -1626,45 +1628,45 @@ __global__ void __launch_bounds__(kSelThreads)
         }
         return;
     }
-    SrcCand32 src{cand_key + (int64_t)q * cap, cand_doc + (int64_t)q * cap, (int64_t)n};
-    block_topk<32>(src, k, sh, false);
-    if (!FP) {
+    const SrcCand32 src{cand_key + (int64_t)q * cap, cand_doc + (int64_t)q * cap, (int64_t)n};
+    if constexpr (!FP) {
+        block_topk<uint32_t>(src, k, sh, false);
         for (int i = threadIdx.x; i < k; i += blockDim.x) {
-            reinterpret_cast<int32_t *>(out_scores)[(int64_t)row * k + i] = (int32_t)sh.key[i];
-            out_ids[(int64_t)row * k + i] = (int64_t)sh.doc[i];
+            reinterpret_cast<int32_t *>(out_scores)[(int64_t)row * k + i] = (int32_t)sh.key_at(i);
+            out_ids[(int64_t)row * k + i] = (int64_t)sh.doc_at(i);
         }
         if (threadIdx.x == 0) status[row] = GS_ROW_DONE;
         return;
     }
-    const uint32_t kth = (uint32_t)sh.key[k - 1];
-    const uint32_t mf = mfix[q];
-    if (kth <= mf) {  // k-th score not clear of zero by the margin
-        if (threadIdx.x == 0) {
-            status[row] = GS_ROW_DENSE;
-            resc_cnt[q] = 0;
+    if constexpr (FP) {
+        const SelKeysLds<SrcCand32> keys(src, reinterpret_cast<uint32_t *>(gs_sel_lds), held);
+        const uint32_t kth = (uint32_t)sel_cut(keys, k, 0u, sh, false);
+        const uint32_t mf = mfix[q];
+        if (kth <= mf) {  // k-th score not clear of zero by the margin
+            if (threadIdx.x == 0) {
+                status[row] = GS_ROW_DENSE;
+                resc_cnt[q] = 0;
+            }
+            return;
         }
-        return;
-    }
-    const uint32_t t_low = kth - mf;
-    if (threadIdx.x == 0) s_m = 0;
-    __syncthreads();
-    const uint32_t *ck = cand_key + (int64_t)q * cap;
-    const uint32_t *cd = cand_doc + (int64_t)q * cap;
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        if (ck[i] >= t_low) {
+        const uint32_t t_low = kth - mf;
+        if (threadIdx.x == 0) s_m = 0;
+        __syncthreads();
+        keys.each([&](int64_t i, uint64_t kk) {
+            if ((uint32_t)kk < t_low) return;
             const uint32_t s = atomicAdd(&s_m, 1u);
-            if (s < (uint32_t)resc_cap) resc_doc[(int64_t)q * resc_cap + s] = cd[i];
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t m = s_m;
-        if (m > (uint32_t)resc_cap) {
-            status[row] = GS_ROW_DENSE;
-            resc_cnt[q] = 0;
-        } else {
-            status[row] = GS_ROW_DONE;
-            resc_cnt[q] = m;
+            if (s < (uint32_t)resc_cap) resc_doc[(int64_t)q * resc_cap + s] = src.doc[i];
+        });
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t m = s_m;
+            if (m > (uint32_t)resc_cap) {
+                status[row] = GS_ROW_DENSE;
+                resc_cnt[q] = 0;
+            } else {
+                status[row] = GS_ROW_DONE;
+                resc_cnt[q] = m;
+            }
         }
     }
 }
@@ -1900,7 +1902,7 @@ __global__ void __launch_bounds__(64 * kRescoreWaves, 8)
 }
 
 template <int WT>
-__global__ void __launch_bounds__(kSelThreads)
+__global__ void __launch_bounds__(kSelThreads, 8)
     k_select_final(const uint32_t *__restrict__ resc_doc, const uint64_t *__restrict__ resc_key,
                    const uint32_t *__restrict__ resc_cnt, int32_t resc_cap, int32_t k,
                    const int32_t *__restrict__ perm, const int32_t *__restrict__ status,
@@ -1911,10 +1913,10 @@ __global__ void __launch_bounds__(kSelThreads)
     const int row = perm ? perm[q] : q;  // query: output row
     if (status[row] != GS_ROW_DONE) return;
     SrcCand64 src{resc_key + (int64_t)q * resc_cap, resc_doc + (int64_t)q * resc_cap, (int64_t)resc_cnt[q]};
-    block_topk<64>(src, k, sh, false);
+    block_topk<uint64_t>(src, k, sh, false);
     for (int i = threadIdx.x; i < k; i += blockDim.x) {
-        out_scores[(int64_t)row * k + i] = (float)gs_unkey_f64(sh.key[i]);
-        out_ids[(int64_t)row * k + i] = (int64_t)sh.doc[i];
+        out_scores[(int64_t)row * k + i] = (float)gs_unkey_f64(sh.key_at(i));
+        out_ids[(int64_t)row * k + i] = (int64_t)sh.doc_at(i);
     }
 }
 
@@ -1930,17 +1932,17 @@ __global__ void __launch_bounds__(kSelThreads)
     const int q = rows ? rows[r0 + r] : r0 + r;
     if (WT == GS_W_U8) {
         SrcRowU32 src{reinterpret_cast<const uint32_t *>(dense) + (int64_t)r * ld, n_docs};
-        block_topk<32>(src, k, sh, false);
+        block_topk<uint32_t>(src, k, sh, false);
         for (int i = threadIdx.x; i < k; i += blockDim.x) {
-            reinterpret_cast<int32_t *>(out_scores)[(int64_t)q * k + i] = (int32_t)sh.key[i];
-            out_ids[(int64_t)q * k + i] = (int64_t)sh.doc[i];
+            reinterpret_cast<int32_t *>(out_scores)[(int64_t)q * k + i] = (int32_t)sh.key_at(i);
+            out_ids[(int64_t)q * k + i] = (int64_t)sh.doc_at(i);
         }
     } else {
         SrcRowF64 src{reinterpret_cast<const double *>(dense) + (int64_t)r * ld, n_docs};
-        block_topk<64>(src, k, sh, false);
+        block_topk<uint64_t>(src, k, sh, false);
         for (int i = threadIdx.x; i < k; i += blockDim.x) {
-            reinterpret_cast<float *>(out_scores)[(int64_t)q * k + i] = (float)gs_unkey_f64(sh.key[i]);
-            out_ids[(int64_t)q * k + i] = (int64_t)sh.doc[i];
+            reinterpret_cast<float *>(out_scores)[(int64_t)q * k + i] = (float)gs_unkey_f64(sh.key_at(i));
+            out_ids[(int64_t)q * k + i] = (int64_t)sh.doc_at(i);
         }
     }
 }
@@ -1962,17 +1964,17 @@ __global__ void __launch_bounds__(kSelThreads)
                          false};
     for (int done = 0; done < k;) {
         const int kr = min(kMaxK, k - done);
-        const int got = block_topk<64>(src, kr, sh, true);  // == kr: k <= n_docs
+        const int got = block_topk<uint64_t>(src, kr, sh, true);  // == kr: k <= n_docs
         for (int i = threadIdx.x; i < got; i += blockDim.x) {
-            const uint64_t key = sh.key[i] - 1;
+            const uint64_t key = sh.key_at(i) - 1;
             const int64_t o = (int64_t)q * k + done + i;
             if (F64) reinterpret_cast<float *>(out_scores)[o] = (float)gs_unkey_f64(key);
             else reinterpret_cast<int32_t *>(out_scores)[o] = (int32_t)(uint32_t)key;
-            out_ids[o] = (int64_t)sh.doc[i];
+            out_ids[o] = (int64_t)sh.doc_at(i);
         }
         if (got <= 0) break;
-        src.ck = sh.key[got - 1] - 1;
-        src.cd = sh.doc[got - 1];
+        src.ck = sh.key_at(got - 1) - 1;
+        src.cd = sh.doc_at(got - 1);
         src.cut = true;
         done += got;
         __syncthreads();  // the next round rewrites the sort buffer
@@ -2349,9 +2351,15 @@ int search_impl(const gs_index *ix, const int32_t *qt, const void *qw, int32_t B
 
     // 3. selection (+ fp64 rescoring for float weights)
     const size_t sel_lds = sel_lds_bytes(k);
-    GS_CHECK_HIP(sel_attr((const void *)k_select_cands<WT>, sel_lds));
-    k_select_cands<WT><<<B, kSelThreads, sel_lds, s>>>(p.cand_doc, p.cand_key, p.cnt, p.cap, k, p.mfix, p.resc_doc,
-                                                 p.resc_cnt, p.rcap, perm, out_scores, out_ids, status);
+    // Float rows keep their keys in LDS instead of a sort buffer: up to one row per
+    // CU a row may fill it (a small batch emits tens of thousands of candidates per
+    // row), with more rows than CUs two of them share a CU.
+    const int held = (int)std::min<int64_t>(p.cap, (B <= kCus ? 144 * 1024 : 64 * 1024) / 4);
+    const size_t cand_lds = FP ? (size_t)held * 4 : sel_lds;
+    GS_CHECK_HIP(sel_attr((const void *)k_select_cands<WT>, cand_lds));
+    k_select_cands<WT><<<B, kSelThreads, cand_lds, s>>>(p.cand_doc, p.cand_key, p.cnt, p.cap, k, held, p.mfix,
+                                                        p.resc_doc, p.resc_cnt, p.rcap, perm, out_scores, out_ids,
+                                                        status);
     GS_CHECK_LAUNCH();
     if ((rc = phase(5))) return rc;
     if (FP) {
