@@ -59,7 +59,6 @@ constexpr int64_t kSeedMaxTiles = 64;       // most tiles of a default seed wide
 constexpr int64_t kPairMinWgs = 12288;    // workgroups (~48 per CU) needed before a workgroup scores two tiles
 constexpr int64_t kTripleMinWgs = 49152;  // and before it scores three
 constexpr int kCus = 256;  // compute units of the GPU
-constexpr size_t kTileLds = 144 * 1024;  // LDS of the fp64 / uint32 row tiles of one dense-path workgroup
 // LDS of the score slices of one fused-scoring workgroup (2 queries x 8192 docs):
 // two such workgroups share a CU, so one's set-up and emission (latency-bound)
 // overlap the other's adds
@@ -252,95 +251,340 @@ __device__ __forceinline__ uint32_t packed_contrib(uint32_t qv, uint32_t word) {
     return (uint32_t)__mul24((int32_t)qv, (int32_t)word >> 16);
 }
 
-// ---------------------------------------------------------------------- dense per-query tiles
+// ---------------------------------------------------------------------- dense per-query rows
 
 struct DenseArgs {
     const int32_t *doc;
     const void *w;
     const int64_t *offsets;
     const int32_t *tb;  // [V][n_tiles + 1]
+    const float *max_abs;
+    const int32_t *dup;
     const int32_t *qt;
     const void *qw;
     const int32_t *rows;  // optional row -> query map
     int64_t n_docs;
     int32_t V, T, R, tile_log2, n_tiles;
-    int32_t tile_begin, tiles, groups, per_xcd;
+    int32_t sub_log2;       // docs per wave and pass: at most kDenseSub, within a tile
+    int32_t blocks;         // workgroups per row
+    int32_t per_xcd;
     void *dense;
-    int64_t dense_ld, dense_col0;
+    int64_t dense_ld;
+    float *scale;    // [R] bin scale of each row, or null: no histogram wanted
+    uint32_t *hist;  // [R][GS_HIST_BINS] docs per score bin (bin 0 not counted)
 };
 
-// One wave owns one (query, tile): it walks the query's terms in order, adds
-// every posting of the tile into its LDS slice and writes the slice to a dense
-// row: fp64 for float weights (terms added in query order, i.e. the fp64
-// scatter-add itself) or uint32 for uint8 impacts -- the exact dense path.
-template <int WT, int UNROLL>
-__global__ void __launch_bounds__(512) k_score_dense(const DenseArgs a) {
+constexpr int kDenseSub = 256;    // docs of one wave's LDS slice
+constexpr int kDenseWaves = 4;    // waves per workgroup, one row
+constexpr int kDenseAhead = 4;    // terms whose postings are loaded together
+constexpr int kDenseBlocks = 1024;  // most workgroups per row (each flushes its histogram once)
+
+// Bin of a dense score: positive scores times the row's scale (2^31 / an upper
+// bound on |score|), as gs_bin_of; everything else, and every score of a row
+// without a finite bound (scale 0), in bin 0.  Monotone in the score.
+__device__ __forceinline__ uint32_t dense_bin(double v, float scale) {
+    return v > 0.0 && scale > 0.0f ? gs_bin_of((float)v * scale) : 0u;
+}
+
+// Exact scores of one row (query) at a time: fp64 sums for float weights (terms
+// added in query order, i.e. the fp64 scatter-add itself) or uint32 for uint8
+// impacts, written to the dense row; with `hist` also the docs per score bin.
+// A wave owns 256 docs of a row and walks the query's terms in order: lane j finds
+// term j's postings of those docs (the tile's bounds, then a four-way search with
+// both ends' probes in flight together), the postings of four terms are loaded
+// while the previous four are added, and a list that holds each doc once is added
+// with plain LDS reads and writes: no other wave writes the slice, and a
+// ds_add_f64 sustains 0.26 lane-adds per clock and CU where a read and a write of
+// 8 bytes sustain several.  Lists with repeated docs take the atomic.
+// What bounds it is latency at one query (the chain bounds -> postings -> adds) and
+// the instructions per (term, 256 docs) at many: about 40 us plus 20 to 27 us per
+// million (query, doc) pairs.  Scores of one query on 100K / 1M docs 425 -> 37 and
+// 515 -> 73 us, of 256 queries on 100K docs 1610 -> ~600, against 16384-doc slices
+// of one wave per CU.  (Fewer workgroups per row, so that a batch of rows fills the
+// chip once, left it to the longest query: 64 queries on 100K docs 184 -> 288 us.)
+template <int WT>
+__global__ void __launch_bounds__(64 * kDenseWaves, 4) k_score_dense(const DenseArgs a) {
     using W = gs_weight<WT>;
     using store_t = typename W::store_t;
     constexpr bool kF64 = WT != GS_W_U8;
     using acc_t = typename std::conditional<kF64, double, uint32_t>::type;
+    constexpr int U = kDenseSub / 64;
 
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int waves = (int)(blockDim.x >> 6);
+    __shared__ acc_t s_acc[kDenseWaves][kDenseSub];
+    __shared__ uint32_t s_hist[GS_HIST_BINS];
     const int wave = gs_uniform((int)(threadIdx.x >> 6));
     const int lane = gs_lane();
 
     // XCD-aware block order: workgroup i runs on XCD i % 8; each XCD gets a
-    // contiguous run of (tile, query group) pairs, query groups fastest.
+    // contiguous run of (block of docs, row) pairs, rows fastest, so that the rows of
+    // a batch share a block's postings in that XCD's L2.
     const int64_t lin = (int64_t)(blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
-    if (lin >= (int64_t)a.tiles * a.groups) return;
-    const int tile = a.tile_begin + (int)(lin / a.groups);
-    const int r = (int)(lin % a.groups) * waves + wave;
-    if (r >= a.R) return;
+    if (lin >= (int64_t)a.blocks * a.R) return;
+    const int blk = (int)(lin / a.R);
+    const int r = (int)(lin % a.R);
     const int q = a.rows ? gs_uniform(a.rows[r]) : r;
 
-    const int TILE = 1 << a.tile_log2;
-    acc_t *acc = reinterpret_cast<acc_t *>(lds_raw) + (size_t)wave * TILE;
-    for (int i = lane; i < TILE; i += 64) acc[i] = (acc_t)0;
-
-    const int64_t doc0 = (int64_t)tile << a.tile_log2;
+    if (a.hist) {
+        for (int i = threadIdx.x; i < GS_HIST_BINS; i += 64 * kDenseWaves) s_hist[i] = 0;
+        __syncthreads();
+    }
+    acc_t *acc = s_acc[wave];
     const int32_t *qt = a.qt + (int64_t)q * a.T;
     const int64_t row = (int64_t)a.n_tiles + 1;
     const store_t *wall = reinterpret_cast<const store_t *>(a.w);
-    for (int j = 0; j < a.T; ++j) {
-        const int32_t t = qt[j];
-        if ((uint32_t)t >= (uint32_t)a.V) continue;
-        const int32_t *bt = a.tb + (int64_t)t * row + tile;
-        const int lo = bt[0], hi = bt[1];
-        if (lo >= hi) continue;
-        const int64_t base = a.offsets[t];
-        const int32_t *dp = a.doc + base;
-        const store_t *wp = wall + base;
-        uint32_t qbits = 0;
-        double wq64 = 0.0;
-        if (WT == GS_W_U8)
-            qbits = reinterpret_cast<const uint8_t *>(a.qw)[(int64_t)q * a.T + j];
-        else
-            wq64 = (double)reinterpret_cast<const float *>(a.qw)[(int64_t)q * a.T + j];
-        auto contrib = [&](store_t wv) -> acc_t {
-            if (kF64) return (acc_t)(wq64 * (double)W::decode(wv));
-            return (acc_t)fixed_contrib<WT>(qbits, wv);
-        };
-        int p = lo + lane;
-        const int nfull = (hi - lo) / (64 * UNROLL);
-        for (int it = 0; it < nfull; ++it, p += 64 * UNROLL) {
-            int32_t d[UNROLL];
-            store_t wv[UNROLL];
+    const int sub_docs = 1 << a.sub_log2;
+    const int64_t n_sub = (a.n_docs + sub_docs - 1) >> a.sub_log2;
+    // a row's subs go to its workgroups in runs of kDenseWaves, one per wave
+    for (int64_t sub = (int64_t)blk * kDenseWaves + wave; sub < n_sub; sub += (int64_t)a.blocks * kDenseWaves) {
+        const int64_t d0 = sub << a.sub_log2;
+        const int64_t d1 = d0 + sub_docs;
+        const int tile = (int)(d0 >> a.tile_log2);
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                d[u] = dp[p + 64 * u];
-                wv[u] = wp[p + 64 * u];
+        for (int u = 0; u < U; ++u) acc[u * 64 + lane] = (acc_t)0;
+        gs_wave_sync();
+        double M = 0.0;  // bound on |score|: sum |q| max|w| (1 + repeats)
+        for (int j0 = 0; j0 < a.T; j0 += 64) {
+            const int j = j0 + lane;
+            const int32_t t = j < a.T ? qt[j] : -1;
+            int n_l = 0, rep_l = 0;
+            int64_t base_l = 0;
+            double q_l = 0.0;
+            uint32_t qi_l = 0;
+            if ((uint32_t)t < (uint32_t)a.V) {
+                const int32_t *bt = a.tb + (int64_t)t * row + tile;
+                int lo = bt[0], hi = bt[1];
+                base_l = a.offsets[t];
+                rep_l = a.dup[t];
+                if (kF64) q_l = (double)reinterpret_cast<const float *>(a.qw)[(int64_t)q * a.T + j];
+                else qi_l = reinterpret_cast<const uint8_t *>(a.qw)[(int64_t)q * a.T + j];
+                M += (kF64 ? fabs(q_l) : (double)qi_l) * (double)a.max_abs[t] * (1.0 + (double)rep_l);
+                const int32_t *dp = a.doc + base_l;
+                // first postings at or past d0 and d1 (ends of the tile are known)
+                int l1 = lo, h1 = (d0 & ((1ll << a.tile_log2) - 1)) == 0 ? lo : hi;
+                int l2 = (d1 & ((1ll << a.tile_log2) - 1)) == 0 ? hi : lo, h2 = hi;
+                while (l1 < h1 || l2 < h2) {
+                    const int s1 = h1 - l1, s2 = h2 - l2;
+                    // three probes of each range; an ended range probes in bounds, unused
+                    const int e1 = max(hi - 1, lo), a1 = min(l1 + (s1 >> 2), e1), b1 = min(l1 + (s1 >> 1), e1),
+                              c1 = min(l1 + s1 - 1 - (s1 >> 2), e1);
+                    const int a2 = min(l2 + (s2 >> 2), e1), b2 = min(l2 + (s2 >> 1), e1),
+                              c2 = min(l2 + s2 - 1 - (s2 >> 2), e1);
+                    const int32_t va1 = dp[max(a1, lo)], vb1 = dp[max(b1, lo)], vc1 = dp[max(c1, lo)];
+                    const int32_t va2 = dp[max(a2, lo)], vb2 = dp[max(b2, lo)], vc2 = dp[max(c2, lo)];
+                    if (l1 < h1) {
+                        if (vb1 < d0) {
+                            if (c1 > b1 && vc1 < d0) l1 = c1 + 1;
+                            else {
+                                l1 = b1 + 1;
+                                if (c1 > b1) h1 = c1;
+                            }
+                        } else if (a1 < b1 && va1 >= d0) h1 = a1;
+                        else {
+                            h1 = b1;
+                            if (a1 < b1) l1 = a1 + 1;
+                        }
+                    }
+                    if (l2 < h2) {
+                        if (vb2 < d1) {
+                            if (c2 > b2 && vc2 < d1) l2 = c2 + 1;
+                            else {
+                                l2 = b2 + 1;
+                                if (c2 > b2) h2 = c2;
+                            }
+                        } else if (a2 < b2 && va2 >= d1) h2 = a2;
+                        else {
+                            h2 = b2;
+                            if (a2 < b2) l2 = a2 + 1;
+                        }
+                    }
+                }
+                base_l += l1;
+                n_l = l2 - l1;
             }
+            struct Stage {
+                int n, rep;
+                double q;
+                uint32_t qi;
+                int64_t base;
+                int32_t d[U];
+                store_t w[U];
+            };
+            // the term of lane l (l < 0: none, which loads one valid posting and adds nothing)
+            auto fetch = [&](int l, int any, Stage &s) {
+                const int ll = l < 0 ? any : l;
+                s.base = gs_readlane_i64(base_l, ll);
+                s.n = l < 0 ? 0 : __builtin_amdgcn_readlane(n_l, ll);
+                s.rep = __builtin_amdgcn_readlane(rep_l, ll);
+                if (kF64) s.q = gs_readlane_f64(q_l, ll);
+                else s.qi = (uint32_t)__builtin_amdgcn_readlane((int)qi_l, ll);
+                const int last = max(s.n - 1, 0);
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) lds_add<acc_t>(acc + (int)(d[u] - doc0), contrib(wv[u]));
+                for (int u = 0; u < U; ++u) {
+                    const int i = min(u * 64 + lane, last);
+                    s.d[u] = a.doc[s.base + i];
+                    s.w[u] = wall[s.base + i];
+                }
+            };
+            auto contrib = [&](const Stage &s, store_t wv) -> acc_t {
+                if constexpr (kF64) return (acc_t)(s.q * (double)W::decode(wv));
+                else return (acc_t)__umul24(s.qi, (uint32_t)wv);
+            };
+            auto apply = [&](const Stage &s) {
+                if (s.n == 0) return;
+                if (s.rep) {  // repeated docs: atomics, in list order, any number of postings
+                    for (int i = lane; i < s.n; i += 64)
+                        lds_add<acc_t>(acc + (int)(a.doc[s.base + i] - d0), contrib(s, wall[s.base + i]));
+                    gs_wave_sync();
+                    return;
+                }
+                // each doc once, so at most 256 postings, and no two of them share a word:
+                // all reads, then all writes (lanes past the end read a word of the list)
+                gs_dispatch_upto<U>((s.n + 63) >> 6, [&](auto ngc) {
+                    constexpr int NG = decltype(ngc)::value;
+                    acc_t v[NG];
+#pragma unroll
+                    for (int u = 0; u < NG; ++u) v[u] = acc[(int)(s.d[u] - d0)] + contrib(s, s.w[u]);
+#pragma unroll
+                    for (int u = 0; u < NG; ++u)
+                        if (u * 64 + lane < s.n) acc[(int)(s.d[u] - d0)] = v[u];
+                });
+                gs_wave_sync();
+            };
+            uint64_t live = __ballot(n_l > 0);
+            if (!live) continue;
+            const int any = __ffsll((unsigned long long)live) - 1;
+            auto next = [&]() {
+                if (!live) return -1;
+                const int l = __ffsll((unsigned long long)live) - 1;
+                live &= live - 1;
+                return l;
+            };
+            Stage cur[kDenseAhead], nxt[kDenseAhead];
+#pragma unroll
+            for (int s = 0; s < kDenseAhead; ++s) fetch(next(), any, cur[s]);
+            while (true) {
+                const bool more = live != 0;
+                if (more)
+#pragma unroll
+                    for (int s = 0; s < kDenseAhead; ++s) fetch(next(), any, nxt[s]);
+#pragma unroll
+                for (int s = 0; s < kDenseAhead; ++s) apply(cur[s]);
+                if (!more) break;
+#pragma unroll
+                for (int s = 0; s < kDenseAhead; ++s) cur[s] = nxt[s];
+            }
         }
-        for (; p < hi; p += 64) lds_add<acc_t>(acc + (int)(dp[p] - doc0), contrib(wp[p]));
+        float scale = 0.0f;
+        if (a.hist) {
+#pragma unroll
+            for (int d = 32; d >= 1; d >>= 1) M += __shfl_xor(M, d, 64);
+            scale = M > 0.0 && M < 0x1p120 ? (float)(0x1p31 / fmax(M, 0x1p-90)) : 0.0f;
+            if (sub == 0 && lane == 0) a.scale[r] = scale;
+        }
+        acc_t *out = reinterpret_cast<acc_t *>(a.dense) + (int64_t)r * a.dense_ld + d0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = u * 64 + lane;
+            if (i < sub_docs && d0 + i < a.n_docs) {
+                const acc_t v = acc[i];
+                out[i] = v;
+                if (a.hist) {
+                    const uint32_t b = dense_bin((double)v, scale);
+                    if (b) atomicAdd(&s_hist[b], 1u);
+                }
+            }
+        }
+        gs_wave_sync();
     }
+    if (!a.hist) return;
+    __syncthreads();
+    uint32_t *h = a.hist + (int64_t)r * GS_HIST_BINS;
+    for (int i = threadIdx.x; i < GS_HIST_BINS; i += 64 * kDenseWaves)
+        if (s_hist[i]) atomicAdd(h + i, s_hist[i]);
+}
 
-    const int64_t left = a.n_docs - doc0;
-    const int ncols = left < TILE ? (int)left : TILE;
-    acc_t *out = reinterpret_cast<acc_t *>(a.dense) + (int64_t)r * a.dense_ld + (doc0 - a.dense_col0);
-    for (int i = lane; i < ncols; i += 64) out[i] = acc[i];
+// Candidates of a dense row: every doc in the highest bins that together hold at
+// least k docs (all docs when the positive bins hold fewer), listed for the exact
+// selection; a row with more than `cap` of them gets cnt = 2^32 - 1 and is selected from in
+// full.  One pass over the row by many workgroups, 4096 docs each, with one slot
+// reservation each, in place of ten passes by the row's one selecting workgroup.
+template <int WT>
+__global__ void __launch_bounds__(256)
+    k_dense_cands(const void *__restrict__ dense, int64_t ld, int64_t n_docs, int32_t k,
+                  const float *__restrict__ scale, const uint32_t *__restrict__ hist, int32_t cap,
+                  uint64_t *__restrict__ cand_key, uint32_t *__restrict__ cand_doc, uint32_t *__restrict__ cnt) {
+    constexpr bool kF64 = WT != GS_W_U8;
+    using acc_t = typename std::conditional<kF64, double, uint32_t>::type;
+    constexpr int PER = 16;
+    __shared__ uint32_t s_wave[4], s_bin, s_tot, s_cnt[4], s_base;
+    const int r = blockIdx.y;
+    const int tid = threadIdx.x, lane = gs_lane();
+    const int wave = gs_uniform(tid >> 6);
+    const acc_t *rowp = reinterpret_cast<const acc_t *>(dense) + (int64_t)r * ld;
+    const float sc = scale[r];
+    const int64_t i0 = blockIdx.x * (int64_t)(256 * PER) + tid;
+    acc_t v[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int64_t i = i0 + u * 256;
+        v[u] = i < n_docs ? rowp[i] : (acc_t)0;
+    }
+    // thread i holds bins 2047 - 8i .. 2040 - 8i, counted from the top
+    const uint32_t *h = hist + (int64_t)r * GS_HIST_BINS;
+    static_assert(GS_HIST_BINS == 8 * 256, "eight bins per thread");
+    if (tid == 0) {
+        s_bin = 0;
+        s_tot = (uint32_t)n_docs;
+    }
+    uint32_t c[8], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += (c[j] = h[GS_HIST_BINS - 1 - 8 * tid - j]);
+    const uint32_t inc = gs_wave_incl_scan(sum);
+    if (lane == 63) s_wave[wave] = inc;
+    __syncthreads();
+    uint32_t before = inc - sum;
+    for (int w = 0; w < wave; ++w) before += s_wave[w];
+    if (before < (uint32_t)k && before + sum >= (uint32_t)k) {  // one thread at most
+        int j = 0;
+        while (before + c[j] < (uint32_t)k) before += c[j++];
+        s_bin = (uint32_t)(GS_HIST_BINS - 1 - 8 * tid - j);
+        s_tot = before + c[j];
+    }
+    __syncthreads();
+    const uint32_t bin = s_bin;
+    if (s_tot > (uint32_t)cap) {
+        if (blockIdx.x == 0 && tid == 0) cnt[r] = 0xFFFFFFFFu;
+        return;
+    }
+    uint64_t m[PER];
+    uint32_t n = 0;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        m[u] = __ballot(i0 + u * 256 < n_docs && dense_bin((double)v[u], sc) >= bin);
+        n += (uint32_t)__popcll(m[u]);
+    }
+    if (lane == 0) s_cnt[wave] = n;
+    __syncthreads();
+    if (tid == 0) {
+        const uint32_t tot = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+        s_base = tot ? atomicAdd(cnt + r, tot) : 0u;
+    }
+    __syncthreads();
+    uint32_t at = s_base;
+    for (int w = 0; w < wave; ++w) at += s_cnt[w];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        if (m[u] >> lane & 1ull) {
+            const uint32_t slot = at + (uint32_t)__popcll(m[u] & gs_lanemask_lt());
+            if (slot < (uint32_t)cap) {
+                const int64_t o = (int64_t)r * cap + slot;
+                if constexpr (kF64) cand_key[o] = gs_key_f64(v[u]);
+                else cand_key[o] = v[u];
+                cand_doc[o] = (uint32_t)(i0 + u * 256);
+            }
+        }
+        at += (uint32_t)__popcll(m[u]);
+    }
 }
 
 // ---------------------------------------------------------------------- query-group unions
@@ -1920,30 +2164,33 @@ __global__ void __launch_bounds__(kSelThreads, 8)
     }
 }
 
-// Dense rows (fp64 or uint32) -> exact top-k.
+// Dense rows (fp64 or uint32) -> exact top-k, from the row's candidates
+// (k_dense_cands; cnt null: none were listed) or from the whole row.
 template <int WT>
 __global__ void __launch_bounds__(kSelThreads)
     k_select_dense(const void *__restrict__ dense, int64_t ld, int64_t n_docs, int32_t k,
-                   const int32_t *__restrict__ rows, int32_t r0, void *__restrict__ out_scores,
-                   int64_t *__restrict__ out_ids) {
+                   const int32_t *__restrict__ rows, int32_t r0, const uint64_t *__restrict__ cand_key,
+                   const uint32_t *__restrict__ cand_doc, const uint32_t *__restrict__ cnt, int32_t cap,
+                   void *__restrict__ out_scores, int64_t *__restrict__ out_ids) {
     __shared__ SelStatic sst;
     SelShared sh = sel_view(sst, k);
     const int r = blockIdx.x;
     const int q = rows ? rows[r0 + r] : r0 + r;
-    if (WT == GS_W_U8) {
+    const uint32_t n = cnt ? cnt[r] : 0xFFFFFFFFu;
+    if (n <= (uint32_t)cap) {
+        SrcCand64 src{cand_key + (int64_t)r * cap, cand_doc + (int64_t)r * cap, (int64_t)n};
+        block_topk<uint64_t>(src, k, sh, false);
+    } else if constexpr (WT == GS_W_U8) {
         SrcRowU32 src{reinterpret_cast<const uint32_t *>(dense) + (int64_t)r * ld, n_docs};
         block_topk<uint32_t>(src, k, sh, false);
-        for (int i = threadIdx.x; i < k; i += blockDim.x) {
-            reinterpret_cast<int32_t *>(out_scores)[(int64_t)q * k + i] = (int32_t)sh.key_at(i);
-            out_ids[(int64_t)q * k + i] = (int64_t)sh.doc_at(i);
-        }
     } else {
         SrcRowF64 src{reinterpret_cast<const double *>(dense) + (int64_t)r * ld, n_docs};
         block_topk<uint64_t>(src, k, sh, false);
-        for (int i = threadIdx.x; i < k; i += blockDim.x) {
-            reinterpret_cast<float *>(out_scores)[(int64_t)q * k + i] = (float)gs_unkey_f64(sh.key_at(i));
-            out_ids[(int64_t)q * k + i] = (int64_t)sh.doc_at(i);
-        }
+    }
+    for (int i = threadIdx.x; i < k; i += blockDim.x) {
+        if (WT == GS_W_U8) reinterpret_cast<int32_t *>(out_scores)[(int64_t)q * k + i] = (int32_t)sh.key_at(i);
+        else reinterpret_cast<float *>(out_scores)[(int64_t)q * k + i] = (float)gs_unkey_f64(sh.key_at(i));
+        out_ids[(int64_t)q * k + i] = (int64_t)sh.doc_at(i);
     }
 }
 
@@ -1983,37 +2230,18 @@ __global__ void __launch_bounds__(kSelThreads)
 
 // ---------------------------------------------------------------------- host plumbing
 
-int dense_waves(int tile_log2, size_t acc_bytes) {
-    const size_t per = (size_t(1) << tile_log2) * acc_bytes;
-    int w = (int)(kTileLds / per);
-    if (w > 8) w = 8;
-    return w;
-}
-
-template <int WT, int UNROLL>
-int launch_dense_u(DenseArgs a, int waves, size_t acc_bytes, hipStream_t s) {
-    static std::atomic<bool> attr_set{false};
-    auto fn = k_score_dense<WT, UNROLL>;
-    const size_t lds = (size_t)waves * (size_t(1) << a.tile_log2) * acc_bytes;
-    if (!attr_set.load()) {
-        GS_CHECK_HIP(allow_full_lds((const void *)fn));
-        attr_set.store(true);
-    }
-    a.groups = (a.R + waves - 1) / waves;
-    const int64_t total = (int64_t)a.tiles * a.groups;
+template <int WT>
+int launch_dense(DenseArgs a, hipStream_t s) {
+    const int64_t n_sub = (a.n_docs + (1ll << a.sub_log2) - 1) >> a.sub_log2;
+    a.blocks = (int32_t)std::min<int64_t>((n_sub + kDenseWaves - 1) / kDenseWaves, kDenseBlocks);
+    const int64_t total = (int64_t)a.blocks * a.R;
     if (total == 0) return GS_OK;
     a.per_xcd = (int32_t)((total + 7) / 8);
     const int64_t grid = (int64_t)a.per_xcd * 8;
     GS_REQUIRE(grid < 0x7FFFFFFFll, "scoring grid too large (%lld workgroups)", (long long)grid);
-    fn<<<(unsigned)grid, waves * 64, lds, s>>>(a);
+    k_score_dense<WT><<<(unsigned)grid, 64 * kDenseWaves, 0, s>>>(a);
     GS_CHECK_LAUNCH();
     return GS_OK;
-}
-
-template <int WT>
-int launch_dense(DenseArgs a, int waves, hipStream_t s) {
-    constexpr size_t acc_bytes = WT != GS_W_U8 ? 8 : 4;
-    return launch_dense_u<WT, 4>(a, waves, acc_bytes, s);
 }
 
 template <int WT, int UNROLL, bool HD>
@@ -2200,6 +2428,8 @@ DenseArgs dense_args(const gs_index *ix, const int32_t *qt, const void *qw, int3
     a.w = ix->weights_d;
     a.offsets = ix->offsets_d;
     a.tb = ix->tile_bounds_d;
+    a.max_abs = ix->max_abs_d;
+    a.dup = ix->dup_d;
     a.qt = qt;
     a.qw = qw;
     a.n_docs = ix->n_docs;
@@ -2207,7 +2437,26 @@ DenseArgs dense_args(const gs_index *ix, const int32_t *qt, const void *qw, int3
     a.T = T;
     a.tile_log2 = ix->tile_log2;
     a.n_tiles = ix->n_tiles;
+    a.sub_log2 = std::min(ix->tile_log2, 8);
+    static_assert(kDenseSub == 1 << 8, "docs per wave");
     return a;
+}
+
+// One row of the dense path's workspace: the scores, and for k <= kMaxK the
+// score bins, their scale, the candidates and their count.
+constexpr int kDenseCandMin = 16384;  // fewest candidate slots per row
+struct DenseRow {
+    int64_t score_bytes;  // of the dense scores
+    int32_t cap;          // candidate slots
+    size_t bytes;         // of everything
+};
+DenseRow dense_row(const gs_index *ix, size_t acc_bytes) {
+    DenseRow d;
+    d.score_bytes = (int64_t)ix->n_tiles * (1ll << ix->tile_log2) * (int64_t)acc_bytes;
+    d.cap = (int32_t)std::min<int64_t>((int64_t)ix->n_tiles << ix->tile_log2, std::max(kDenseCandMin, 2 * kMaxK));
+    // + 256: the arrays of a pass start 256-byte aligned, whatever its rows
+    d.bytes = (size_t)d.score_bytes + (size_t)d.cap * 12 + GS_HIST_BINS * 4 + 8 + 5 * 256;
+    return d;
 }
 
 template <int WT>
@@ -2394,36 +2643,56 @@ int search_dense_impl(const gs_index *ix, const int32_t *qt, const void *qw, int
                       const int32_t *rows, int32_t R, void *out_scores, int64_t *out_ids, void *ws, size_t ws_bytes,
                       hipStream_t s) {
     constexpr size_t acc_bytes = WT == GS_W_U8 ? 4 : 8;
-    const int64_t TILE = 1ll << ix->tile_log2;
-    const int64_t ld = (int64_t)ix->n_tiles * TILE;
-    const int64_t per_row = ld * (int64_t)acc_bytes;
-    const int64_t rows_per_pass = (int64_t)(ws_bytes / (size_t)per_row);
+    const int64_t ld = (int64_t)ix->n_tiles << ix->tile_log2;
+    const DenseRow dr = dense_row(ix, acc_bytes);
+    // A workspace without room for one row's candidates still holds its scores: the
+    // rows are then selected from in full.
+    const bool listed = k <= kMaxK && ws_bytes >= dr.bytes;
+    // (at most 32768 rows: they are a grid's y dimension)
+    const int64_t rows_per_pass =
+        std::min<int64_t>(32768, (int64_t)(ws_bytes / (listed ? dr.bytes : (size_t)dr.score_bytes)));
     if (rows_per_pass < 1) {
-        gs_set_error("dense workspace too small: one row needs %lld bytes, got %zu", (long long)per_row, ws_bytes);
+        gs_set_error("dense workspace too small: one row needs %lld bytes, got %zu", (long long)dr.score_bytes,
+                     ws_bytes);
         return GS_ENOSPC;
     }
-    const int waves = dense_waves(ix->tile_log2, acc_bytes);
     for (int32_t r0 = 0; r0 < R; r0 += (int32_t)rows_per_pass) {
         const int32_t n = (int32_t)std::min<int64_t>(rows_per_pass, R - r0);
         DenseArgs a = dense_args(ix, qt, qw, T);
         a.rows = rows ? rows + r0 : nullptr;
         a.R = n;
-        a.tile_begin = 0;
-        a.tiles = ix->n_tiles;
         a.dense = ws;
         a.dense_ld = ld;
-        a.dense_col0 = 0;
+        uint64_t *cand_key = nullptr;
+        uint32_t *cand_doc = nullptr, *cnt = nullptr;
+        if (listed) {
+            gs_arena ar{reinterpret_cast<char *>(ws), (size_t)dr.score_bytes * n, ws_bytes};
+            a.hist = ar.take<uint32_t>((size_t)n * (GS_HIST_BINS + 1));  // and the counts, cleared with it
+            cnt = a.hist + (size_t)n * GS_HIST_BINS;
+            a.scale = ar.take<float>(n);
+            cand_key = ar.take<uint64_t>((size_t)n * dr.cap);
+            cand_doc = ar.take<uint32_t>((size_t)n * dr.cap);
+            GS_REQUIRE(ar.ok(), "dense workspace accounting");
+            const int64_t words = (int64_t)n * (GS_HIST_BINS + 1);
+            k_fill<uint32_t><<<gs_blocks(words, 256, 4096), 256, 0, s>>>(a.hist, words, 0u);
+            GS_CHECK_LAUNCH();
+        }
         // rows == nullptr means queries r0..r0+n-1: shift the query pointers
         if (!rows) {
             a.qt = qt + (int64_t)r0 * T;
             a.qw = reinterpret_cast<const char *>(qw) + (int64_t)r0 * T * (WT == GS_W_U8 ? 1 : 4);
         }
-        int rc = launch_dense<WT>(a, waves, s);
+        int rc = launch_dense<WT>(a, s);
         if (rc) return rc;
         if (k <= kMaxK) {
+            if (listed) {
+                k_dense_cands<WT><<<dim3(gs_blocks(ix->n_docs, 4096), (unsigned)n), 256, 0, s>>>(
+                    ws, ld, ix->n_docs, k, a.scale, a.hist, dr.cap, cand_key, cand_doc, cnt);
+                GS_CHECK_LAUNCH();
+            }
             GS_CHECK_HIP(sel_attr((const void *)k_select_dense<WT>, sel_lds_bytes(k)));
-            k_select_dense<WT><<<n, kSelThreads, sel_lds_bytes(k), s>>>(ws, ld, ix->n_docs, k, rows, r0,
-                                                                         out_scores, out_ids);
+            k_select_dense<WT><<<n, kSelThreads, sel_lds_bytes(k), s>>>(ws, ld, ix->n_docs, k, rows, r0, cand_key,
+                                                                         cand_doc, cnt, dr.cap, out_scores, out_ids);
         } else {
             GS_CHECK_HIP(sel_attr((const void *)k_select_dense_large<WT>, sel_lds_bytes(kMaxK)));
             k_select_dense_large<WT><<<n, kSelThreads, sel_lds_bytes(kMaxK), s>>>(ws, ld, ix->n_docs, k, rows, r0,
@@ -2578,8 +2847,7 @@ extern "C" int gs_search_noalloc(const gs_index *index, const int32_t *q_terms_d
 extern "C" int gs_search_dense_workspace(const gs_index *index, int32_t rows_per_pass, size_t *bytes) {
     if (int rc = check_index(index)) return rc;
     GS_REQUIRE(rows_per_pass > 0 && bytes, "bad arguments");
-    const size_t acc = index->wtype == GS_W_U8 ? 4 : 8;
-    *bytes = (size_t)rows_per_pass * (size_t)index->n_tiles * ((size_t)1 << index->tile_log2) * acc;
+    *bytes = (size_t)rows_per_pass * dense_row(index, index->wtype == GS_W_U8 ? 4 : 8).bytes;
     return GS_OK;
 }
 

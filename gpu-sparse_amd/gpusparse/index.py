@@ -405,7 +405,8 @@ def build_head(index):
     return head, rank
 
 
-def ensure_search_state(index, tile_log2: int | None = None, forward: bool = True, hybrid: bool = False) -> dict:
+def ensure_search_state(index, tile_log2: int | None = None, forward: bool = True, hybrid: bool = False,
+                        scorer: bool = True) -> dict:
     """Derived arrays gs_search needs: max |w|, duplicate counts, the most frequent
     terms (query grouping), tile bounds, the
     packed scoring copy for this tile size (skipped when the GPU has no room for it
@@ -415,7 +416,8 @@ def ensure_search_state(index, tile_log2: int | None = None, forward: bool = Tru
     `forward` is false or the GPU has no room for it: the rescoring then searches
     the term lists, with the same results).  With `hybrid` also the heavy terms'
     dense copy (skipped when it does not fit: the search then adds every term in
-    LDS, with the same results)."""
+    LDS, with the same results).  Without `scorer` only what the dense path reads:
+    max |w|, duplicate counts and tile bounds."""
     if tile_log2 is None:
         tile_log2 = default_tile_log2(index)
     a = index.aux()
@@ -426,7 +428,7 @@ def ensure_search_state(index, tile_log2: int | None = None, forward: bool = Tru
     if "dup" not in a:
         require_ascending(index)
     list_max_abs(index)
-    if "heavy" not in a:
+    if scorer and "heavy" not in a:
         a["heavy"] = heavy_terms(index)
     key = ("tile_bounds", tile_log2)
     if key not in a:
@@ -437,7 +439,7 @@ def ensure_search_state(index, tile_log2: int | None = None, forward: bool = Tru
                                     N, tile_log2, _lib.ptr(tb), _lib.stream_ptr(dev)), "gs_tile_bounds")
         a[key] = tb
     key = ("packed", tile_log2)
-    if key not in a and int(index.doc_ids.numel()) > 0:
+    if scorer and key not in a and int(index.doc_ids.numel()) > 0:
         # One word per posting (4 of 8, 6 or 5 bytes).  One packed copy per index:
         # the one for the tile size last searched.
         for old in [k for k in a if isinstance(k, tuple) and k[0] == "packed"]:
@@ -451,7 +453,7 @@ def ensure_search_state(index, tile_log2: int | None = None, forward: bool = Tru
             a["head"] = build_head(index)
         except torch.cuda.OutOfMemoryError:
             a["head"] = None
-    if forward and "fwd" not in a and index.wtype != _lib.GS_W_U8 and int(index.num_docs) > 0:
+    if scorer and forward and "fwd" not in a and index.wtype != _lib.GS_W_U8 and int(index.num_docs) > 0:
         try:
             a["fwd"] = build_forward(index)
         except torch.cuda.OutOfMemoryError:
@@ -514,12 +516,12 @@ def build_packed(index, tile_log2: int, arrange: bool = True) -> Packed | None:
     return Packed(out, shift)
 
 
-def gs_index_struct(index, tile_log2: int | None = None, hybrid: bool = False) -> _lib.GsIndex:
+def gs_index_struct(index, tile_log2: int | None = None, hybrid: bool = False, scorer: bool = True) -> _lib.GsIndex:
     """The C view of the index for tile_log2; with `hybrid` it carries the heavy
-    terms' dense copy as well."""
+    terms' dense copy as well, without `scorer` at least what the dense path reads."""
     if tile_log2 is None:
         tile_log2 = default_tile_log2(index)
-    a = ensure_search_state(index, tile_log2, hybrid=hybrid)
+    a = ensure_search_state(index, tile_log2, hybrid=hybrid, scorer=scorer)
     N = int(index.num_docs)
     s = _lib.GsIndex()
     s.doc_ids_d = index.doc_ids.data_ptr()
@@ -538,7 +540,9 @@ def gs_index_struct(index, tile_log2: int | None = None, hybrid: bool = False) -
     fwd = a.get("fwd")
     if fwd is not None:
         s.fwd_ptr_d, s.fwd_terms_d, s.fwd_weights_d = (t.data_ptr() for t in fwd)
-    s.heavy_d = a["heavy"].data_ptr()
+    heavy = a.get("heavy")
+    if heavy is not None:
+        s.heavy_d = heavy.data_ptr()
     pk = a.get(("packed", tile_log2))
     if pk is not None:
         s.packed_d, s.packed_tile_log2, s.packed_shift = pk.words.data_ptr(), tile_log2, pk.shift

@@ -208,6 +208,25 @@ def _dense_rows(index, gidx, qt, qw, k, rows, out_s, out_i, dense_budget):
                "gs_search_dense")
 
 
+DENSE_PAIRS = 3 << 20     # (query, doc) pairs up to which a batch's dense rows are the faster path ...
+DENSE_PAIRS_PER_K = 4096  # ... and further pairs per result asked for
+
+
+def dense_preferred(index, B: int, k: int, tile_log2: int, hybrid: bool, dense_budget: int) -> bool:
+    """Whether path "auto" scores a batch of B queries as dense rows: when the rows
+    fit `dense_budget` and the batch has at most DENSE_PAIRS + DENSE_PAIRS_PER_K k
+    (query, doc) pairs.  Dense rows take four launches and ~25 us per million
+    pairs; the fused path takes ten launches, few us per million pairs and, in a
+    small batch, time that grows with k (its threshold starts low).  Dense against
+    fused, us: 16 queries on 100K docs k = 10 82 / 127, k = 1000 102 / 199; 64 on
+    100K 184 / 148 and 206 / 225; 4 on 1M 199 / 148 and 223 / 494; 16 on 1M 501 /
+    168 and 546 / 339; 1 on 4M 136 / 252 and 158 / 572."""
+    docs = -(-int(index.num_docs) >> tile_log2) << tile_log2
+    acc_bytes = 4 if index.wtype == _lib.GS_W_U8 and not hybrid else 8
+    return B * docs * acc_bytes <= dense_budget and \
+        B * int(index.num_docs) <= DENSE_PAIRS + DENSE_PAIRS_PER_K * k
+
+
 class PendingSearch:
     """A search whose kernels are queued on a stream (`search_async`).
 
@@ -260,7 +279,8 @@ def search(index, query_batch, k: int = 10, *, tile_log2: int | None = None, pat
     hybrid: the index's heavy (64 longest) lists as int8 matrix products, the other terms
     as LDS adds (scorer_choice; a uint8 index through its float16 copy); results
     are the same either way.
-    path: "auto" (dense when the [B, N] rows fit `dense_budget`), "fused" or "dense";
+    path: "auto" (dense for small batches whose [B, N] rows fit `dense_budget`,
+    dense_preferred), "fused" or "dense";
     k above MAX_K (8192) or queries wider than MAX_T (8192 terms) always take the
     dense path (any k up to the doc count, any width).
     timing: optional dict; receives event pairs on the launch stream bracketing the
@@ -304,6 +324,25 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         qw = torch.zeros((B, 1), dtype=qw.dtype, device=dev)
         T = 1
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
+    if path not in ("auto", "fused", "dense"):
+        raise ValueError(f"unknown path {path!r}")
+    stream = torch.cuda.current_stream(dev)
+    # k above MAX_K or queries wider than MAX_T terms: the dense path, whose
+    # selection takes any k (rounds of MAX_K) and whose scorer any width
+    if path == "dense" or kk > MAX_K or T > MAX_T or (path == "auto" and dense_preferred(index, B, kk, tile_log2, hyb,
+                                                                                        dense_budget)):
+        late = hyb and index.wtype == _lib.GS_W_U8  # the weights' check is read with the results
+        if bad_w is not None and not late and bool(bad_w):
+            raise ValueError(_U8_WEIGHTS_MSG)
+        gidx = gs_index_struct(index, tile_log2, scorer=False)
+        _dense_rows(index, gidx, qt, qw, kk, None, out_s, out_i, max(dense_budget, 1))
+
+        def checked(out):
+            if bool(bad_w):
+                raise ValueError(_U8_WEIGHTS_MSG)
+            return out
+
+        return PendingSearch((out_s, out_i), stream, post=checked if late and bad_w is not None else None)
     if hyb and index.wtype == _lib.GS_W_U8:
         # the float16 copy's hybrid search; its fp32 scores are the exact sums.
         # The weights' check (device weights) is copied out ahead of the search,
@@ -312,7 +351,7 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         if bad_w is not None:
             bad_h = torch.empty((), dtype=torch.bool, pin_memory=True)
             bad_h.copy_(bad_w, non_blocking=True)
-        inner = search_async(u8_float_copy(index), (qt, qw.to(torch.float32)), k, tile_log2=tile_log2, path=path,
+        inner = search_async(u8_float_copy(index), (qt, qw.to(torch.float32)), k, tile_log2=tile_log2, path="fused",
                              sample_tiles=sample_tiles, cand_cap=cand_cap, unroll=unroll, waves=waves,
                              tiles_per_wg=tiles_per_wg, dense_budget=dense_budget, timing=timing,
                              batch_order=batch_order, hybrid=True)
@@ -326,19 +365,6 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         return inner
     gidx = gs_index_struct(index, tile_log2, hyb)
     L = _lib.lib()
-    acc_bytes = 4 if index.scores.dtype == torch.uint8 else 8
-    dense_bytes = B * gidx.n_tiles * (1 << tile_log2) * acc_bytes
-    if path not in ("auto", "fused", "dense"):
-        raise ValueError(f"unknown path {path!r}")
-    stream = torch.cuda.current_stream(dev)
-    # k above MAX_K or queries wider than MAX_T terms: the dense path, whose
-    # selection takes any k (rounds of MAX_K) and whose scorer any width
-    use_dense = path == "dense" or kk > MAX_K or T > MAX_T or (path == "auto" and dense_bytes <= dense_budget)
-    if use_dense:
-        if bad_w is not None and bool(bad_w):
-            raise ValueError(_U8_WEIGHTS_MSG)
-        _dense_rows(index, gidx, qt, qw, kk, None, out_s, out_i, max(dense_budget, 1))
-        return PendingSearch((out_s, out_i), stream)
     opts = _opts(sample_tiles, cand_cap, unroll, waves, tiles_per_wg, batch_order, hyb)
     need = _lib.C.c_size_t()
     _lib.check(L.gs_search_workspace(_lib.C.byref(gidx), B, T, kk, _lib.C.byref(opts), _lib.C.byref(need)),
