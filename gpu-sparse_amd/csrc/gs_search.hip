@@ -2228,6 +2228,8 @@ __global__ void __launch_bounds__(kSelThreads)
     }
 }
 
+#include "gs_blocks.h"
+
 // ---------------------------------------------------------------------- host plumbing
 
 template <int WT>
@@ -2343,6 +2345,17 @@ bool hybrid_usable(const gs_index *ix, const gs_search_opts *o) {
     return ix->wtype != GS_W_U8 && packed_usable(ix);
 }
 
+// Candidate slots per query: kCandBudget of them spread over the batch, as small
+// batches emit more candidates per query (their tiles are scored all at once, and
+// tau rises little after the seed); a query cannot emit more candidates than
+// there are docs.
+int cand_slots(const gs_index *ix, int32_t B, int32_t k, const gs_search_opts *o) {
+    if (o && o->cand_cap > 0) return std::max(o->cand_cap, 2 * k);
+    int64_t c = std::max<int64_t>(kDefaultCandCap, std::min<int64_t>(kMaxCandCap, kCandBudget / B));
+    c = std::min<int64_t>(c, (ix->n_docs + 255) / 256 * 256);
+    return std::max((int)c, 2 * k);
+}
+
 SearchPlan plan_search(const gs_index *ix, int32_t B, int32_t T, int32_t k, const gs_search_opts *o,
                        gs_arena &ar) {
     SearchPlan p;
@@ -2372,17 +2385,7 @@ SearchPlan plan_search(const gs_index *ix, int32_t B, int32_t T, int32_t k, cons
     s_def = std::max<int64_t>(s_def, std::min<int64_t>(kSeedMaxTiles, (kSeedFillWgs + p.n_groups - 1) / p.n_groups));
     p.S = (o && o->sample_tiles > 0) ? o->sample_tiles : (int)s_def;
     if (p.S > ix->n_tiles) p.S = ix->n_tiles;
-    if (o && o->cand_cap > 0) {
-        p.cap = o->cand_cap;
-    } else {
-        // kCandBudget slots spread over the batch, as small batches emit more
-        // candidates per query (the same reason as above); a query cannot emit
-        // more candidates than there are docs
-        int64_t c = std::max<int64_t>(kDefaultCandCap, std::min<int64_t>(kMaxCandCap, kCandBudget / B));
-        c = std::min<int64_t>(c, (ix->n_docs + 255) / 256 * 256);
-        p.cap = (int)c;
-    }
-    if (p.cap < 2 * k) p.cap = 2 * k;
+    p.cap = cand_slots(ix, B, k, o);
     p.rcap = kRescoreCap;
     // default postings per lane per chunk: 16 on packed one-word postings (their
     // registers allow it), else 8
@@ -2457,6 +2460,53 @@ DenseRow dense_row(const gs_index *ix, size_t acc_bytes) {
     // + 256: the arrays of a pass start 256-byte aligned, whatever its rows
     d.bytes = (size_t)d.score_bytes + (size_t)d.cap * 12 + GS_HIST_BINS * 4 + 8 + 5 * 256;
     return d;
+}
+
+// Selection (+ fp64 rescoring for float weights) of the emitted candidates of a
+// batch, whichever scorer emitted them.
+template <int WT, class Plan, class Phase>
+int select_and_rescore(const gs_index *ix, const int32_t *qt, const void *qw, int32_t B, int32_t T, int32_t k,
+                       const Plan &p, const int32_t *perm, void *out_scores, int64_t *out_ids, int32_t *status,
+                       Phase &&phase, hipStream_t s) {
+    constexpr bool FP = WT != GS_W_U8;
+    int rc = GS_OK;
+    const size_t sel_lds = sel_lds_bytes(k);
+    // Float rows keep their keys in LDS instead of a sort buffer: up to one row per
+    // CU a row may fill it (a small batch emits tens of thousands of candidates per
+    // row), with more rows than CUs two of them share a CU.
+    const int held = (int)std::min<int64_t>(p.cap, (B <= kCus ? 144 * 1024 : 64 * 1024) / 4);
+    const size_t cand_lds = FP ? (size_t)held * 4 : sel_lds;
+    GS_CHECK_HIP(sel_attr((const void *)k_select_cands<WT>, cand_lds));
+    k_select_cands<WT><<<B, kSelThreads, cand_lds, s>>>(p.cand_doc, p.cand_key, p.cnt, p.cap, k, held, p.mfix,
+                                                        p.resc_doc, p.resc_cnt, p.rcap, perm, out_scores, out_ids,
+                                                        status);
+    GS_CHECK_LAUNCH();
+    if ((rc = phase(5))) return rc;
+    if (FP) {
+        dim3 g(64u, (unsigned)B);
+        // doc-major rescoring: about 16K waves over the batch (16 to 64 workgroups
+        // per query), so that each wave's start-up is spread over more candidates
+        // (C2: 0.51 -> 0.48 ms at 16 per query); small batches keep 64 per query
+        const dim3 gf((unsigned)std::min(64, std::max(16, (16384 / kRescoreWaves) / std::max(B, 1))), (unsigned)B);
+        if (ix->fwd_ptr_d)
+            k_rescore_fwd<WT><<<gf, 64 * kRescoreWaves, 0, s>>>(
+                ix->fwd_ptr_d, ix->fwd_terms_d, ix->fwd_weights_d, ix->vocab, qt,
+                reinterpret_cast<const float *>(qw), T, p.resc_doc, p.resc_cnt, p.rcap, p.resc_key);
+        else
+            k_rescore<WT><<<g, 256, 0, s>>>(ix->doc_ids_d, ix->weights_d, ix->offsets_d, ix->tile_bounds_d,
+                                            ix->vocab, ix->n_tiles, ix->tile_log2, qt,
+                                            reinterpret_cast<const float *>(qw), T, p.resc_doc, p.resc_cnt, p.rcap,
+                                            p.resc_key);
+        GS_CHECK_LAUNCH();
+    }
+    if ((rc = phase(6))) return rc;
+    if (FP) {
+        GS_CHECK_HIP(sel_attr((const void *)k_select_final<WT>, sel_lds));
+        k_select_final<WT><<<B, kSelThreads, sel_lds, s>>>(p.resc_doc, p.resc_key, p.resc_cnt, p.rcap, k, perm,
+                                                           status, reinterpret_cast<float *>(out_scores), out_ids);
+        GS_CHECK_LAUNCH();
+    }
+    return GS_OK;
 }
 
 template <int WT>
@@ -2598,43 +2648,217 @@ int search_impl(const gs_index *ix, const int32_t *qt, const void *qw, int32_t B
     }
     if ((rc = phase(4))) return rc;
 
-    // 3. selection (+ fp64 rescoring for float weights)
-    const size_t sel_lds = sel_lds_bytes(k);
-    // Float rows keep their keys in LDS instead of a sort buffer: up to one row per
-    // CU a row may fill it (a small batch emits tens of thousands of candidates per
-    // row), with more rows than CUs two of them share a CU.
-    const int held = (int)std::min<int64_t>(p.cap, (B <= kCus ? 144 * 1024 : 64 * 1024) / 4);
-    const size_t cand_lds = FP ? (size_t)held * 4 : sel_lds;
-    GS_CHECK_HIP(sel_attr((const void *)k_select_cands<WT>, cand_lds));
-    k_select_cands<WT><<<B, kSelThreads, cand_lds, s>>>(p.cand_doc, p.cand_key, p.cnt, p.cap, k, held, p.mfix,
-                                                        p.resc_doc, p.resc_cnt, p.rcap, perm, out_scores, out_ids,
-                                                        status);
+    if ((rc = select_and_rescore<WT>(ix, qt, qw, B, T, k, p, perm, out_scores, out_ids, status, phase, s))) return rc;
+    return phase(7);
+}
+
+// ---------------------------------------------------------------------- block search
+
+constexpr int64_t kBlkSeedDocs = 16384;  // docs of the block search's first threshold (more for large k)
+constexpr int64_t kBlkGrowth = 2;        // docs known after a scoring launch, per doc before it (1M docs, 512
+                                         // queries, k = 1000: 1233 / 1250 / 1263 us at 2 / 3 / 4)
+constexpr int kBlkList = 16384;          // emitted scores a workgroup's list holds
+
+struct BlkPlan {
+    int32_t chunks, Q, slots, seed_docs, cap, rcap;
+    int64_t ent_ld;
+    float *scale;
+    uint32_t *mfix, *tau, *cnt, *cand_doc, *cand_key, *resc_doc, *resc_cnt;
+    uint64_t *resc_key;
+    int8_t *alimb;
+    int32_t *shift, *kq;
+    double *ct;
+    uint2 *tab;
+    uint64_t *live;
+    uint32_t *total, *ent, *seed, *out_q, *out_doc, *out_key, *out_n;
+    int64_t cleared;  // 32-bit words from tab on that each search clears (tab, total)
+    int32_t lists;    // scoring workgroups, all chunks
+};
+
+BlkPlan plan_blocks(const gs_index *ix, const gs_block_copy *bk, int32_t B, int32_t T, int32_t k,
+                    const gs_search_opts *o, gs_arena &ar) {
+    BlkPlan p{};
+    // chunks of up to kBlkMaxQ queries, evenly filled
+    p.chunks = (B + kBlkMaxQ - 1) / kBlkMaxQ;
+    p.Q = ((B + p.chunks - 1) / p.chunks + 15) & ~15;
+    p.slots = p.chunks * p.Q;
+    // Docs scored in full for the first threshold: its docs' share of the top k sets
+    // how many docs of the first blocks become candidates, so 16 per result, at most
+    // kBlkSeedDocs, but four per result at least; at most an eighth of a small collection beyond those.
+    int64_t sd = std::max<int64_t>(std::min<int64_t>(std::max<int64_t>(16ll * k, 4096), kBlkSeedDocs), 4ll * k);
+    sd = std::min<int64_t>(sd, std::max<int64_t>(ix->n_docs / 8, 4ll * k));
+    sd = (std::min<int64_t>(sd, ix->n_docs) + kBlkDocs - 1) / kBlkDocs * kBlkDocs;
+    p.seed_docs = (int32_t)sd;
+    p.cap = cand_slots(ix, B, k, o);
+    p.rcap = kRescoreCap;
+    p.ent_ld = (int64_t)p.Q * T + 8;  // + 8: entries are read four and eight at a time
+    p.mfix = ar.take<uint32_t>(B);
+    p.tau = ar.take<uint32_t>(B);
+    p.cnt = ar.take<uint32_t>(B);
+    p.resc_cnt = ar.take<uint32_t>(B);
+    p.cleared = (int64_t)p.chunks * (bk->n_tail + 1) * 2 + p.chunks;
+    uint32_t *cleared = ar.take<uint32_t>((size_t)p.cleared);
+    p.tab = reinterpret_cast<uint2 *>(cleared);
+    p.total = cleared ? cleared + (size_t)(p.cleared - p.chunks) : nullptr;
+    // two workgroups per CU over all chunks
+    p.lists = std::max(1, 2 * kCus / p.chunks) * p.chunks;
+    p.out_q = ar.take<uint32_t>((size_t)p.lists * kBlkList);
+    p.out_doc = ar.take<uint32_t>((size_t)p.lists * kBlkList);
+    p.out_key = ar.take<uint32_t>((size_t)p.lists * kBlkList);
+    p.out_n = ar.take<uint32_t>((size_t)p.lists);
+    p.live = ar.take<uint64_t>((size_t)p.chunks * blk_live_words(bk->n_tail));
+    p.ent = ar.take<uint32_t>((size_t)(p.chunks * p.ent_ld));
+    p.cand_doc = ar.take<uint32_t>((size_t)B * p.cap);
+    p.cand_key = ar.take<uint32_t>((size_t)B * p.cap);
+    p.resc_doc = ar.take<uint32_t>((size_t)B * p.rcap);
+    p.resc_key = ar.take<uint64_t>((size_t)B * p.rcap);
+    p.alimb = ar.take<int8_t>((size_t)p.slots * 2 * kBlkHeavy);
+    p.shift = ar.take<int32_t>(p.slots);
+    p.kq = ar.take<int32_t>(p.slots);
+    p.ct = ar.take<double>(p.slots);
+    p.seed = ar.take<uint32_t>((size_t)p.slots * p.seed_docs);
+    return p;
+}
+
+int check_blocks(const gs_index *ix, const gs_block_copy *bk) {
+    GS_REQUIRE(ix && bk, "null index or blocks");
+    GS_REQUIRE(ix->wtype == GS_W_F32 || ix->wtype == GS_W_F16, "the block search takes float weights, got type %d",
+               ix->wtype);
+    GS_REQUIRE(ix->vocab > 0 && ix->n_docs > 0 && ix->n_docs < 0x7FFFFFFFll, "bad index sizes");
+    GS_REQUIRE(ix->max_abs_d && ix->dup_d && ix->fwd_ptr_d && ix->fwd_terms_d && ix->fwd_weights_d,
+               "the block search reads the doc-major copy, max |w| and the repeat counts");
+    GS_REQUIRE(bk->head_d && bk->tail_d && bk->count_d && bk->rank_d && bk->heavy_d, "blocks have a null device array");
+    GS_REQUIRE(bk->levels == 255 || bk->levels == 127, "levels %d, not 255 or 127", bk->levels);
+    GS_REQUIRE(bk->n_tail >= 1 && bk->n_tail <= 65535, "n_tail %d outside [1, 65535]", bk->n_tail);
+    return GS_OK;
+}
+
+template <int WT>
+int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_t *qt, const float *qw, int32_t B,
+                       int32_t T, int32_t k, const gs_search_opts *o, float *out_scores, int64_t *out_ids,
+                       int32_t *status, void *ws, size_t ws_bytes, hipStream_t s) {
+    gs_arena ar{reinterpret_cast<char *>(ws), 0, ws_bytes};
+    const BlkPlan p = plan_blocks(ix, bk, B, T, k, o, ar);
+    if (!ar.ok()) {
+        gs_set_error("search workspace too small: need %zu bytes, got %zu", ar.used, ws_bytes);
+        return GS_ENOSPC;
+    }
+    auto phase = [&](int i) -> int {
+        if (o && o->ev_phases && o->ev_phases[i])
+            GS_CHECK_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(o->ev_phases[i]), s));
+        return GS_OK;
+    };
+    int rc = phase(0);
+    if (rc) return rc;
+    k_fill<uint32_t><<<gs_blocks(p.cleared, 256, 4096), 256, 0, s>>>(reinterpret_cast<uint32_t *>(p.tab), p.cleared, 0u);
     GS_CHECK_LAUNCH();
-    if ((rc = phase(5))) return rc;
-    if (FP) {
-        dim3 g(64u, (unsigned)B);
-        // doc-major rescoring: about 16K waves over the batch (16 to 64 workgroups
-        // per query), so that each wave's start-up is spread over more candidates
-        // (C2: 0.51 -> 0.48 ms at 16 per query); small batches keep 64 per query
-        const dim3 gf((unsigned)std::min(64, std::max(16, (16384 / kRescoreWaves) / std::max(B, 1))), (unsigned)B);
-        if (ix->fwd_ptr_d)
-            k_rescore_fwd<WT><<<gf, 64 * kRescoreWaves, 0, s>>>(
-                ix->fwd_ptr_d, ix->fwd_terms_d, ix->fwd_weights_d, ix->vocab, qt,
-                reinterpret_cast<const float *>(qw), T, p.resc_doc, p.resc_cnt, p.rcap, p.resc_key);
-        else
-            k_rescore<WT><<<g, 256, 0, s>>>(ix->doc_ids_d, ix->weights_d, ix->offsets_d, ix->tile_bounds_d,
-                                            ix->vocab, ix->n_tiles, ix->tile_log2, qt,
-                                            reinterpret_cast<const float *>(qw), T, p.resc_doc, p.resc_cnt, p.rcap,
-                                            p.resc_key);
-        GS_CHECK_LAUNCH();
+    BlkQueries bq{};
+    bq.qt = qt;
+    bq.qw = qw;
+    bq.B = B;
+    bq.T = T;
+    bq.V = ix->vocab;
+    bq.Q = p.Q;
+    bq.slots = p.slots;
+    bq.n_tail = bk->n_tail;
+    bq.rank = bk->rank_d;
+    bq.heavy = bk->heavy_d;
+    bq.dup = ix->dup_d;
+    bq.max_abs = ix->max_abs_d;
+    bq.levels = bk->levels;
+    bq.alimb = p.alimb;
+    bq.shift = p.shift;
+    bq.kq = p.kq;
+    bq.ct = p.ct;
+    bq.tab = p.tab;
+    bq.ent = p.ent;
+    bq.ent_ld = p.ent_ld;
+    bq.total = p.total;
+    bq.mfix = p.mfix;
+    bq.tau = p.tau;
+    bq.cnt = p.cnt;
+    k_blk_prep<<<gs_blocks((int64_t)p.slots * 64, 256), 256, 0, s>>>(bq);
+    GS_CHECK_LAUNCH();
+    k_blk_ranges<<<dim3(gs_blocks(bk->n_tail, 1024), (unsigned)p.chunks), 1024, 0, s>>>(p.tab, bk->n_tail, p.total,
+                                                                                           p.live);
+    GS_CHECK_LAUNCH();
+    k_blk_entries<<<gs_blocks((int64_t)B * T, 256, 4096), 256, 0, s>>>(bq);
+    GS_CHECK_LAUNCH();
+    if ((rc = phase(1))) return rc;
+    if ((rc = phase(2))) return rc;
+
+    static std::atomic<bool> attr{false};
+    if (!attr.load()) {
+        GS_CHECK_HIP(allow_full_lds((const void *)k_blk_score<true>));
+        GS_CHECK_HIP(allow_full_lds((const void *)k_blk_score<false>));
+        attr.store(true);
     }
-    if ((rc = phase(6))) return rc;
-    if (FP) {
-        GS_CHECK_HIP(sel_attr((const void *)k_select_final<WT>, sel_lds));
-        k_select_final<WT><<<B, kSelThreads, sel_lds, s>>>(p.resc_doc, p.resc_key, p.resc_cnt, p.rcap, k, perm,
-                                                           status, reinterpret_cast<float *>(out_scores), out_ids);
+    BlkArgs a{};
+    a.head = bk->head_d;
+    a.tail = bk->tail_d;
+    a.count = bk->count_d;
+    a.row_ptr = ix->fwd_ptr_d;
+    a.Q = p.Q;
+    a.B = B;
+    a.chunks = p.chunks;
+    a.n_tail = bk->n_tail;
+    a.alimb = p.alimb;
+    a.shift = p.shift;
+    a.kq = p.kq;
+    a.tab = p.tab;
+    a.ent = p.ent;
+    a.live = p.live;
+    a.ent_ld = p.ent_ld;
+    a.tau = p.tau;
+    a.mfix = p.mfix;
+    a.cnt = p.cnt;
+    a.cand_doc = p.cand_doc;
+    a.cand_key = p.cand_key;
+    a.cap = p.cap;
+    a.out_q = p.out_q;
+    a.out_doc = p.out_doc;
+    a.out_key = p.out_key;
+    a.out_n = p.out_n;
+    a.out_cap = kBlkList;
+    a.collect = blk_collect(p.Q, bk->n_tail);
+    a.seed = p.seed;
+    a.seed_ld = p.seed_docs;
+    const int32_t all = (int32_t)((ix->n_docs + kBlkDocs - 1) / kBlkDocs);
+    auto run = [&](bool seed, int32_t b0, int32_t b1) -> int {
+        a.block0 = b0;
+        a.n_blocks = b1 - b0;
+        a.sets = std::min(a.n_blocks, p.lists / p.chunks);
+        const unsigned grid = (unsigned)((a.sets * p.chunks + 7) / 8 * 8);
+        const size_t lds = blk_lds_fixed(p.Q, bk->n_tail) + (size_t)a.collect * 12;
+        if (seed) k_blk_score<true><<<grid, kBlkThreads, lds, s>>>(a);
+        else k_blk_score<false><<<grid, kBlkThreads, lds, s>>>(a);
         GS_CHECK_LAUNCH();
+        return GS_OK;
+    };
+    if ((rc = run(true, 0, p.seed_docs / kBlkDocs))) return rc;
+    k_blk_tau<<<B, 256, 0, s>>>(p.seed, p.seed_docs, p.seed_docs, nullptr, k, p.tau);
+    GS_CHECK_LAUNCH();
+    if ((rc = phase(3))) return rc;
+    if (o && o->ev_score_begin) GS_CHECK_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(o->ev_score_begin), s));
+    // Every doc again, in launches of kBlkGrowth times the docs scored so far, with the
+    // thresholds raised to the k-th of the candidates in between: a launch emits at most
+    // about kBlkGrowth k scores per query.
+    int64_t known = p.seed_docs / kBlkDocs;
+    for (int32_t b0 = 0; b0 < all;) {
+        const int32_t b1 = (int32_t)std::min<int64_t>(all, std::max<int64_t>(b0 + 1, known * kBlkGrowth));
+        if ((rc = run(false, b0, b1))) return rc;
+        k_blk_deal<<<(unsigned)(a.sets * p.chunks), 512, 0, s>>>(p.out_q, p.out_doc, p.out_key, p.out_n, kBlkList,
+                                                                 p.chunks, p.Q, p.cap, p.cnt, p.cand_doc, p.cand_key);
+        GS_CHECK_LAUNCH();
+        if (b1 < all) {
+            k_blk_tau<<<B, 256, 0, s>>>(p.cand_key, p.cap, p.cap, p.cnt, k, p.tau);
+            GS_CHECK_LAUNCH();
+        }
+        known = b0 = b1;
     }
+    if (o && o->ev_score_end) GS_CHECK_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(o->ev_score_end), s));
+    if ((rc = phase(4))) return rc;
+    if ((rc = select_and_rescore<WT>(ix, qt, qw, B, T, k, p, nullptr, out_scores, out_ids, status, phase, s))) return rc;
     return phase(7);
 }
 
@@ -2790,6 +3014,72 @@ extern "C" int gs_search(const gs_index *index, const int32_t *q_terms_d, const 
     GS_REQUIRE(workspace_d, "null workspace");
     return search_dispatch(index, q_terms_d, q_weights_d, B, T, k, opts, out_scores_d, out_ids_d, status_d,
                            workspace_d, workspace_bytes, gs_stream(stream));
+}
+
+extern "C" int gs_blocks_fill(const int64_t *fwd_ptr_d, const int32_t *fwd_terms_d, const void *fwd_weights_d,
+                              int32_t wtype, int64_t n_docs, int32_t vocab, const int32_t *rank_d,
+                              const float *max_abs_d, int32_t levels, int8_t *head_d, uint32_t *tail_d,
+                              int32_t *count_d, int32_t *negative_d, void *workspace_d, void *stream) {
+    GS_REQUIRE(wtype == GS_W_F32 || wtype == GS_W_F16, "float weights only, got type %d", wtype);
+    GS_REQUIRE(n_docs > 0 && n_docs < 0x7FFFFFFFll && vocab > 0, "bad sizes");
+    GS_REQUIRE(levels == 255 || levels == 127, "levels %d, not 255 or 127", levels);
+    GS_REQUIRE(fwd_ptr_d && fwd_terms_d && fwd_weights_d && rank_d && max_abs_d && head_d && tail_d && count_d &&
+                   negative_d && workspace_d,
+               "null pointer");
+    hipStream_t s = gs_stream(stream);
+    k_fill<int32_t><<<1, 64, 0, s>>>(negative_d, 1, 0);
+    uint2 *info = reinterpret_cast<uint2 *>(workspace_d);
+    k_blk_terms<<<gs_blocks(vocab, 256), 256, 0, s>>>(rank_d, max_abs_d, vocab, levels, info);
+    const unsigned nb = (unsigned)((n_docs + kBlkDocs - 1) / kBlkDocs);
+    if (wtype == GS_W_F32)
+        k_blk_fill<GS_W_F32><<<nb, 512, 0, s>>>(fwd_ptr_d, fwd_terms_d, fwd_weights_d, n_docs, info, levels, head_d,
+                                                tail_d, count_d, negative_d);
+    else
+        k_blk_fill<GS_W_F16><<<nb, 512, 0, s>>>(fwd_ptr_d, fwd_terms_d, fwd_weights_d, n_docs, info, levels, head_d,
+                                                tail_d, count_d, negative_d);
+    GS_CHECK_LAUNCH();
+    return GS_OK;
+}
+
+extern "C" int gs_search_blocks_workspace(const gs_index *index, const gs_block_copy *blocks, int32_t B, int32_t T,
+                                          int32_t k, const gs_search_opts *opts, size_t *bytes) {
+    if (int rc = check_blocks(index, blocks)) return rc;
+    GS_REQUIRE(B > 0 && T > 0 && k > 0 && bytes, "bad search sizes");
+    gs_arena ar{nullptr, 0, 0};
+    plan_blocks(index, blocks, B, T, k, opts, ar);
+    *bytes = ar.used + 256;
+    return GS_OK;
+}
+
+extern "C" int gs_search_blocks(const gs_index *index, const gs_block_copy *blocks, const int32_t *q_terms_d,
+                                const float *q_weights_d, int32_t B, int32_t T, int32_t k, const gs_search_opts *opts,
+                                float *out_scores_d, int64_t *out_ids_d, int32_t *status_d, void *workspace_d,
+                                size_t workspace_bytes, void *stream) {
+    if (int rc = check_blocks(index, blocks)) return rc;
+    GS_REQUIRE(B > 0 && T > 0, "empty query batch (B=%d, T=%d)", B, T);
+    GS_REQUIRE(k >= 1 && k <= kMaxK && (int64_t)k <= index->n_docs, "k=%d outside [1, min(n_docs, %d)]", k, kMaxK);
+    GS_REQUIRE((int64_t)B * T < (1ll << 31), "query batch too large (B=%d, T=%d)", B, T);
+    GS_REQUIRE(q_terms_d && q_weights_d && out_scores_d && out_ids_d && status_d && workspace_d, "null pointer");
+    hipStream_t s = gs_stream(stream);
+    if (index->wtype == GS_W_F32)
+        return search_blocks_impl<GS_W_F32>(index, blocks, q_terms_d, q_weights_d, B, T, k, opts, out_scores_d,
+                                            out_ids_d, status_d, workspace_d, workspace_bytes, s);
+    return search_blocks_impl<GS_W_F16>(index, blocks, q_terms_d, q_weights_d, B, T, k, opts, out_scores_d, out_ids_d,
+                                        status_d, workspace_d, workspace_bytes, s);
+}
+
+extern "C" int gs_search_blocks_counts(const gs_index *index, const gs_block_copy *blocks, int32_t B, int32_t T, int32_t k,
+                                       const gs_search_opts *opts, const void *workspace_d, size_t workspace_bytes,
+                                       uint32_t *cand_d, uint32_t *resc_d, void *stream) {
+    if (int rc = check_blocks(index, blocks)) return rc;
+    GS_REQUIRE(B > 0 && T > 0 && k > 0 && workspace_d && cand_d && resc_d, "bad arguments");
+    gs_arena ar{reinterpret_cast<char *>(const_cast<void *>(workspace_d)), 0, workspace_bytes};
+    const BlkPlan p = plan_blocks(index, blocks, B, T, k, opts, ar);
+    GS_REQUIRE(ar.ok(), "workspace smaller than the search's (%zu < %zu bytes)", workspace_bytes, ar.used);
+    hipStream_t s = gs_stream(stream);
+    GS_CHECK_HIP(hipMemcpyAsync(cand_d, p.cnt, sizeof(uint32_t) * (size_t)B, hipMemcpyDeviceToDevice, s));
+    GS_CHECK_HIP(hipMemcpyAsync(resc_d, p.resc_cnt, sizeof(uint32_t) * (size_t)B, hipMemcpyDeviceToDevice, s));
+    return GS_OK;
 }
 
 // ---------------------------------------------------------------------- allocation-free search

@@ -84,6 +84,24 @@ class GsSearchOpts(C.Structure):
     ]
 
 
+BLOCK_DOCS, BLOCK_HEAVY = 64, 128  # GS_BLOCK_DOCS, GS_BLOCK_HEAVY
+BLOCK_MAX_TAIL = 65535             # most tail terms of a block copy (16-bit ranks)
+
+
+class GsBlockCopy(C.Structure):
+    """Mirror of ``struct gs_block_copy``."""
+
+    _fields_ = [
+        ("head_d", C.c_void_p),
+        ("tail_d", C.c_void_p),
+        ("count_d", C.c_void_p),
+        ("rank_d", C.c_void_p),
+        ("heavy_d", C.c_void_p),
+        ("n_tail", C.c_int32),
+        ("levels", C.c_int32),
+    ]
+
+
 class GsSynthSpec(C.Structure):
     """Mirror of ``gs_synth_spec`` in csrc/synth.c."""
 
@@ -143,6 +161,13 @@ SIGNATURES = {
                                  C.POINTER(GsSearchPlanInfo)]),
     "gs_search": (C.c_int, [C.POINTER(GsIndex), _P, _P, _I32, _I32, _I32, C.POINTER(GsSearchOpts), _P, _P,
                             _P, _P, _SZ, _P]),
+    "gs_blocks_fill": (C.c_int, [_P, _P, _P, _I32, _I64, _I32, _P, _P, _I32, _P, _P, _P, _P, _P, _P]),
+    "gs_search_blocks_workspace": (C.c_int, [C.POINTER(GsIndex), C.POINTER(GsBlockCopy), _I32, _I32, _I32,
+                                             C.POINTER(GsSearchOpts), C.POINTER(_SZ)]),
+    "gs_search_blocks": (C.c_int, [C.POINTER(GsIndex), C.POINTER(GsBlockCopy), _P, _P, _I32, _I32, _I32,
+                                   C.POINTER(GsSearchOpts), _P, _P, _P, _P, _SZ, _P]),
+    "gs_search_blocks_counts": (C.c_int, [C.POINTER(GsIndex), C.POINTER(GsBlockCopy), _I32, _I32, _I32,
+                                          C.POINTER(GsSearchOpts), _P, _SZ, _P, _P, _P]),
     "gs_search_noalloc": (C.c_int, [C.POINTER(GsIndex), _P, _P, _I32, _I32, _I32, C.POINTER(GsSearchOpts), _P, _P,
                                     _P, _P]),
     "gs_search_counts": (C.c_int, [C.POINTER(GsIndex), _I32, _I32, _I32, C.POINTER(GsSearchOpts), _P, _SZ, _P, _P,

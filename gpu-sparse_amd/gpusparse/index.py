@@ -465,6 +465,97 @@ def ensure_search_state(index, tile_log2: int | None = None, forward: bool = Tru
     return a
 
 
+class Blocks(NamedTuple):
+    """The block search's copy of a float index (gs_blocks_fill)."""
+
+    head: torch.Tensor    # int8 [blocks, 64, 128] levels of the heavy terms
+    tail: torch.Tensor    # int32 [postings] words of the other terms, block by block
+    count: torch.Tensor   # int32 [blocks] tail words of each block
+    rank: torch.Tensor    # int32 [vocab] lists by length, -1 for empty ones
+    heavy: torch.Tensor   # int32 [128] term of each heavy rank
+    n_tail: int
+    levels: int           # 255, or 127 when a weight is negative
+
+    def struct(self) -> _lib.GsBlockCopy:
+        return _lib.GsBlockCopy(*(t.data_ptr() for t in self[:5]), self.n_tail, self.levels)
+
+
+def blocks_eligible(index) -> bool:
+    """Whether the block search can serve the index: float weights, all finite, the
+    128 longest lists holding each doc once, at most 65535 further non-empty lists."""
+    a = index.aux()
+    if "blocks_ok" not in a:
+        ok = index.wtype != _lib.GS_W_U8 and int(index.num_docs) > 0
+        if ok:
+            if "dup" not in a:
+                require_ascending(index)
+            # small host copies, no device reduction on the way to the first search
+            length = index.lengths.cpu().numpy()
+            order = np.argsort(-length.astype(np.int64), kind="stable")[:int((length > 0).sum())].astype(np.int32)
+            ok = 0 < order.size <= _lib.BLOCK_HEAVY + _lib.BLOCK_MAX_TAIL and pack_shift(index) is not None and \
+                int(a["dup"].cpu().numpy()[order[:_lib.BLOCK_HEAVY]].max()) == 0
+            if ok:
+                a["block_order"] = order
+        a["blocks_ok"] = bool(ok)
+    return a["blocks_ok"]
+
+
+def ensure_blocks(index) -> Blocks | None:
+    """The block copy of an eligible index and the doc-major copy it is made from,
+    built once; None when the GPU has no room for them (the search then takes the
+    hybrid path, with the same results)."""
+    a = index.aux()
+    if "blocks" in a:
+        return a["blocks"]
+    if not blocks_eligible(index):
+        return None
+    dev = _device_of(index)
+    V, N = int(index.vocab_size), int(index.num_docs)
+    try:
+        if a.get("fwd") is None:
+            a["fwd"] = build_forward(index)
+        ptr, terms, w = a["fwd"]
+        order = a.pop("block_order")
+        rank = np.full(V, -1, dtype=np.int32)
+        rank[order] = np.arange(order.size, dtype=np.int32)
+        heavy = np.full(_lib.BLOCK_HEAVY, -1, dtype=np.int32)
+        heavy[:min(order.size, _lib.BLOCK_HEAVY)] = order[:_lib.BLOCK_HEAVY]
+        rank_d, heavy_d = torch.from_numpy(rank).to(dev), torch.from_numpy(heavy).to(dev)
+        nb = -(-N // _lib.BLOCK_DOCS)
+        head = torch.empty((nb, _lib.BLOCK_DOCS, _lib.BLOCK_HEAVY), dtype=torch.int8, device=dev)
+        tail = torch.empty(max(int(terms.numel()), 1), dtype=torch.int32, device=dev)
+        count = torch.empty(nb, dtype=torch.int32, device=dev)
+        neg = torch.empty(1, dtype=torch.int32, device=dev)
+        ws = torch.empty(V, dtype=torch.int64, device=dev)
+        for levels in (255, 127):
+            _lib.check(_lib.lib().gs_blocks_fill(_lib.ptr(ptr), _lib.ptr(terms), _lib.ptr(w), index.wtype, N, V,
+                                                 _lib.ptr(rank_d), _lib.ptr(list_max_abs(index)), levels,
+                                                 _lib.ptr(head), _lib.ptr(tail), _lib.ptr(count), _lib.ptr(neg),
+                                                 _lib.ptr(ws), _lib.stream_ptr(dev)), "gs_blocks_fill")
+            # reading the flag also completes the copy before a search on another
+            # stream (search_async) reads it
+            if not int(neg.cpu()[0]):
+                break
+        torch.cuda.current_stream(dev).synchronize()
+        a["blocks"] = Blocks(head, tail, count, rank_d, heavy_d, max(order.size - _lib.BLOCK_HEAVY, 1), levels)
+    except torch.cuda.OutOfMemoryError:
+        a["blocks"] = None
+    return a["blocks"]
+
+
+def gs_blocks_index(index) -> _lib.GsIndex:
+    """The C view of an index with a block copy that gs_search_blocks reads."""
+    a = index.aux()
+    s = _lib.GsIndex()
+    s.max_abs_d = list_max_abs(index).data_ptr()
+    s.dup_d = a["dup"].data_ptr()
+    s.n_docs = int(index.num_docs)
+    s.vocab = int(index.vocab_size)
+    s.wtype = index.wtype
+    s.fwd_ptr_d, s.fwd_terms_d, s.fwd_weights_d = (t.data_ptr() for t in a["fwd"])
+    return s
+
+
 def pack_shift(index) -> int | None:
     """Weight scale 2^shift of the packed copy (gs_pack_shift of the largest |w|
     of the index; 0 for uint8), or None when a weight is not finite."""

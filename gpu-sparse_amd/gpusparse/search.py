@@ -21,7 +21,8 @@ import numpy as np
 import torch
 
 from . import _lib
-from .index import DEFAULT_TILE_LOG2_HYBRID, default_tile_log2, gs_index_struct, hybrid_eligible, _device_of
+from .index import (DEFAULT_TILE_LOG2_HYBRID, blocks_eligible, default_tile_log2, ensure_blocks, gs_blocks_index,
+                    gs_index_struct, hybrid_eligible, _device_of)
 
 MAX_K = 8192  # largest k of the fused path and of compacted_topk; search answers larger k densely
 MAX_T = 8192  # widest query batch of the fused path (terms per query); search answers wider ones densely
@@ -227,6 +228,26 @@ def dense_preferred(index, B: int, k: int, tile_log2: int, hybrid: bool, dense_b
         B * int(index.num_docs) <= DENSE_PAIRS + DENSE_PAIRS_PER_K * k
 
 
+BLOCK_MIN_QUERIES = 256    # fewest queries of a batch that takes the block search,
+BLOCK_MIN_PAIRS = 280 << 20  # and its fewest (query, doc) pairs
+
+
+def block_copy(index, B: int, hybrid: bool, default_scorer: bool):
+    """The index's block copy when a fused search of B queries runs on it (built on
+    first use), else None: batches that would take the hybrid search and name neither
+    scorer nor launch shape, of at least BLOCK_MIN_QUERIES and BLOCK_MIN_PAIRS.
+    The block search reads every posting of the collection once per 512 queries,
+    whatever they hold, and scores a query at little more than its products; the
+    hybrid search writes and reads a sum per (query, doc).  Blocks against hybrid,
+    us per batch at k = 1000: 512 queries on 300K docs 819 / 815, on 1M 1235 / 1416,
+    on 8.8M 4980 / 7485; 1024 on 1M 2121 / 2690; 256 on 1M 838 / 838, on 3M 1632 /
+    1715; 200 on 3M 1477 / 1350; 64 on 3M 1094 / 645."""
+    if not (hybrid and default_scorer and B >= BLOCK_MIN_QUERIES and
+            B * int(index.num_docs) >= BLOCK_MIN_PAIRS and blocks_eligible(index)):
+        return None
+    return ensure_blocks(index)
+
+
 class PendingSearch:
     """A search whose kernels are queued on a stream (`search_async`).
 
@@ -323,6 +344,9 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         qt = torch.full((B, 1), -1, dtype=torch.int32, device=dev)
         qw = torch.zeros((B, 1), dtype=qw.dtype, device=dev)
         T = 1
+    default_scorer = hybrid is None and tile_log2 is None and not (sample_tiles or unroll or waves or tiles_per_wg or
+                                                                   batch_order)
+    tile_arg, hybrid_arg = tile_log2, hybrid
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     if path not in ("auto", "fused", "dense"):
         raise ValueError(f"unknown path {path!r}")
@@ -351,10 +375,10 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         if bad_w is not None:
             bad_h = torch.empty((), dtype=torch.bool, pin_memory=True)
             bad_h.copy_(bad_w, non_blocking=True)
-        inner = search_async(u8_float_copy(index), (qt, qw.to(torch.float32)), k, tile_log2=tile_log2, path="fused",
+        inner = search_async(u8_float_copy(index), (qt, qw.to(torch.float32)), k, tile_log2=tile_arg, path="fused",
                              sample_tiles=sample_tiles, cand_cap=cand_cap, unroll=unroll, waves=waves,
                              tiles_per_wg=tiles_per_wg, dense_budget=dense_budget, timing=timing,
-                             batch_order=batch_order, hybrid=True)
+                             batch_order=batch_order, hybrid=hybrid_arg)
 
         def to_int(out):
             if bad_h is not None and bool(bad_h):
@@ -363,12 +387,18 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
 
         inner._post = to_int
         return inner
-    gidx = gs_index_struct(index, tile_log2, hyb)
     L = _lib.lib()
+    ref = _lib.C.byref
     opts = _opts(sample_tiles, cand_cap, unroll, waves, tiles_per_wg, batch_order, hyb)
     need = _lib.C.c_size_t()
-    _lib.check(L.gs_search_workspace(_lib.C.byref(gidx), B, T, kk, _lib.C.byref(opts), _lib.C.byref(need)),
-               "gs_search_workspace")
+    blocks = block_copy(index, B, hyb, default_scorer)
+    if blocks is not None:
+        gidx, bcopy = gs_blocks_index(index), blocks.struct()
+        _lib.check(L.gs_search_blocks_workspace(ref(gidx), ref(bcopy), B, T, kk, ref(opts), ref(need)),
+                   "gs_search_blocks_workspace")
+    else:
+        gidx = gs_index_struct(index, tile_log2, hyb)
+        _lib.check(L.gs_search_workspace(ref(gidx), B, T, kk, ref(opts), ref(need)), "gs_search_workspace")
     ws = _workspace(index, int(need.value), stream.cuda_stream)
     status = torch.empty(B, dtype=torch.int32, device=dev)
     s = _lib.stream_ptr(dev)
@@ -380,9 +410,14 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         opts.ev_score_begin, opts.ev_score_end = evs[0].cuda_event, evs[1].cuda_event
         opts.ev_phases = ph_ptr
         evs[2].record()
-    _lib.check(L.gs_search(_lib.C.byref(gidx), _lib.ptr(qt), _lib.ptr(qw), B, T, kk, _lib.C.byref(opts),
-                           _lib.ptr(out_s), _lib.ptr(out_i), _lib.ptr(status), _lib.ptr(ws), ws.numel(), s),
-               "gs_search")
+    if blocks is not None:
+        _lib.check(L.gs_search_blocks(ref(gidx), ref(bcopy), _lib.ptr(qt), _lib.ptr(qw), B, T, kk, ref(opts),
+                                      _lib.ptr(out_s), _lib.ptr(out_i), _lib.ptr(status), _lib.ptr(ws), ws.numel(), s),
+                   "gs_search_blocks")
+    else:
+        _lib.check(L.gs_search(ref(gidx), _lib.ptr(qt), _lib.ptr(qw), B, T, kk, ref(opts),
+                               _lib.ptr(out_s), _lib.ptr(out_i), _lib.ptr(status), _lib.ptr(ws), ws.numel(), s),
+                   "gs_search")
     if timing is not None:
         evs[3].record()
         timing.setdefault("score_kernel", []).append((evs[0], evs[1]))
@@ -406,7 +441,9 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         if bad.size:
             with torch.cuda.stream(stream):
                 rows = torch.from_numpy(bad.astype(np.int32)).to(dev)
-                _dense_rows(index, gidx, qt, qw, kk, rows, out_s, out_i, max(dense_budget, 1))
+                # (after a block search: the tile bounds are built here, on the first such row)
+                dense_idx = gidx if blocks is None else gs_index_struct(index, tile_log2, scorer=False)
+                _dense_rows(index, dense_idx, qt, qw, kk, rows, out_s, out_i, max(dense_budget, 1))
 
     return PendingSearch((out_s, out_i), stream, done, status_h, finish)
 
@@ -441,9 +478,12 @@ def search_plan(index, B: int, T: int, k: int, *, tile_log2: int | None = None, 
     """How the fused path of `search` runs a batch of B queries of width T
     (gs_search_plan): seed tiles, queries per group, postings per lane per chunk,
     tiles per scoring workgroup, whether the packed copy is read and whether the
-    hybrid scorer runs."""
+    hybrid scorer runs; "blocks": whether the block search runs in its place (the
+    other entries then say what the hybrid scorer would do)."""
+    default_scorer = hybrid is None and tile_log2 is None and not (sample_tiles or unroll or tiles_per_wg or batch_order)
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     index = search_index(index, hyb)
+    blocks = block_copy(index, int(B), hyb, default_scorer)
     gidx = gs_index_struct(index, tile_log2, hyb)
     opts = _opts(sample_tiles, cand_cap, unroll, 0, tiles_per_wg, batch_order, hyb)
     info = _lib.GsSearchPlanInfo()
@@ -451,7 +491,7 @@ def search_plan(index, B: int, T: int, k: int, *, tile_log2: int | None = None, 
                                          _lib.C.byref(opts), _lib.C.byref(info)), "gs_search_plan")
     return {"tile_log2": tile_log2, "seed_tiles": info.seed_tiles, "group_size": info.group_size,
             "unroll": info.unroll, "tiles_per_wg": info.tiles_per_wg, "packed": bool(info.packed),
-            "hybrid": bool(info.hybrid), "cand_cap": info.cand_cap}
+            "hybrid": bool(info.hybrid), "cand_cap": info.cand_cap, "blocks": blocks is not None}
 
 
 def search_counts(index, B: int, T: int, k: int, *, tile_log2: int | None = None, sample_tiles: int = 0,
@@ -460,14 +500,24 @@ def search_counts(index, B: int, T: int, k: int, *, tile_log2: int | None = None
     """Per scoring slot of the fused search that last ran with these arguments:
     (docs the scorer emitted as candidates, candidates rescored in fp64), two
     numpy uint32 [B] arrays (gs_search_counts on the index's cached workspace)."""
+    default_scorer = hybrid is None and tile_log2 is None and not (sample_tiles or unroll or tiles_per_wg or batch_order)
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     index = search_index(index, hyb)
     ws = index.aux().get("workspace")
     if ws is None:
         raise ValueError("no fused search has run on this index")
     dev = _device_of(index)
-    gidx = gs_index_struct(index, tile_log2, hyb)
     opts = _opts(sample_tiles, cand_cap, unroll, 0, tiles_per_wg, batch_order, hyb)
+    blocks = block_copy(index, int(B), hyb, default_scorer)
+    if blocks is not None:
+        gidx, bcopy = gs_blocks_index(index), blocks.struct()
+        cand, resc = (torch.empty(B, dtype=torch.int32, device=dev) for _ in range(2))
+        _lib.check(_lib.lib().gs_search_blocks_counts(_lib.C.byref(gidx), _lib.C.byref(bcopy), int(B), int(T),
+                                                      min(int(k), int(index.num_docs)), _lib.C.byref(opts),
+                                                      _lib.ptr(ws), ws.numel(), _lib.ptr(cand), _lib.ptr(resc),
+                                                      _lib.stream_ptr(dev)), "gs_search_blocks_counts")
+        return cand.cpu().numpy().view(np.uint32), resc.cpu().numpy().view(np.uint32)
+    gidx = gs_index_struct(index, tile_log2, hyb)
     cand = torch.empty(B, dtype=torch.int32, device=dev)
     resc = torch.empty(B, dtype=torch.int32, device=dev)
     _lib.check(_lib.lib().gs_search_counts(_lib.C.byref(gidx), int(B), int(T), min(int(k), int(index.num_docs)),

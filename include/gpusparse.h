@@ -272,6 +272,51 @@ int gs_search(const gs_index *index, const int32_t *q_terms_d, const void *q_wei
               int64_t *out_ids_d, int32_t *status_d, void *workspace_d, size_t workspace_bytes,
               void *stream);
 
+/* ------------------------------------------------------------ block search
+ * No counterpart in the reference: gs_search's answers from a doc-block-major
+ * copy of a float index, for batches of some dozens of queries or more.  Blocks of
+ * GS_BLOCK_DOCS docs; the copy is made from the doc-major copy (gs_forward_fill):
+ *   rank_d   int32 [vocab]: the lists by length, longest first: 0 .. GS_BLOCK_HEAVY - 1
+ *            the heavy terms, GS_BLOCK_HEAVY + x the tail terms x = 0 .. n_tail - 1, -1
+ *            for empty lists (n_tail <= 65535); max_abs_d as in gs_index
+ *   head_d   int8 [blocks][GS_BLOCK_DOCS][GS_BLOCK_HEAVY]: levels rint(w levels / max |w|)
+ *            of the heavy terms, less 128 when levels == 255; within a block doc d,
+ *            term h at byte ((d / 16 * 2 + h / 64) * 64 + h % 64 / 16 * 16 + d % 16) * 16 + h % 16
+ *   tail_d   uint32 [postings], block b's words from fwd_ptr[GS_BLOCK_DOCS b] on, count_d[b]
+ *            of them: level (10 bits, of 511) << 22 | doc in block << 16 | tail rank
+ *   negative_d int32 [1] <- 1 when levels == 255 met a negative weight: the copy is then
+ *            not usable, fill it again with levels = 127
+ *   workspace_d 8 bytes per term of the vocabulary, 8-byte aligned
+ * The heavy lists must hold each doc at most once, and every weight must be finite. */
+#define GS_BLOCK_DOCS 64
+#define GS_BLOCK_HEAVY 128
+typedef struct gs_block_copy {
+    const int8_t *head_d;
+    const uint32_t *tail_d;
+    const int32_t *count_d;
+    const int32_t *rank_d;
+    const int32_t *heavy_d; /* [GS_BLOCK_HEAVY] term of each heavy rank, -1 past the non-empty lists */
+    int32_t n_tail;
+    int32_t levels;         /* 255 or 127 */
+} gs_block_copy;
+int gs_blocks_fill(const int64_t *fwd_ptr_d, const int32_t *fwd_terms_d, const void *fwd_weights_d, int32_t wtype,
+                   int64_t n_docs, int32_t vocab, const int32_t *rank_d, const float *max_abs_d, int32_t levels,
+                   int8_t *head_d, uint32_t *tail_d, int32_t *count_d, int32_t *negative_d, void *workspace_d,
+                   void *stream);
+/* As gs_search (same results, status, phases and score events; of the options only
+ * cand_cap and the events apply).  Of the index it reads n_docs, vocab, wtype,
+ * max_abs_d, dup_d and the doc-major copy. */
+int gs_search_blocks_workspace(const gs_index *index, const gs_block_copy *blocks, int32_t B, int32_t T, int32_t k,
+                               const gs_search_opts *opts, size_t *bytes);
+int gs_search_blocks(const gs_index *index, const gs_block_copy *blocks, const int32_t *q_terms_d,
+                     const float *q_weights_d, int32_t B, int32_t T, int32_t k, const gs_search_opts *opts,
+                     float *out_scores_d, int64_t *out_ids_d, int32_t *status_d, void *workspace_d,
+                     size_t workspace_bytes, void *stream);
+/* gs_search_counts of the gs_search_blocks that last ran on `workspace_d`. */
+int gs_search_blocks_counts(const gs_index *index, const gs_block_copy *blocks, int32_t B, int32_t T, int32_t k,
+                            const gs_search_opts *opts, const void *workspace_d, size_t workspace_bytes,
+                            uint32_t *cand_d, uint32_t *resc_d, void *stream);
+
 /* ------------------------------------------------------------ allocation-free search
  * No counterpart in the reference.  For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that

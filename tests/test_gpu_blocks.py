@@ -1,0 +1,200 @@
+"""The block search (128 heavy terms as int8 products on 64-doc blocks, the other
+terms added in an LDS tile) against the oracle: block, chunk and group edges,
+signs, repeated terms, and its copy's levels and words."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import gpusparse as gs
+import oracle.oracle as O
+from gpusparse import synth
+from gpusparse.index import ensure_blocks
+from gpusparse._lib import BLOCK_HEAVY as H
+from helpers import random_csr, random_queries
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def every_batch(monkeypatch):
+    """Batches of any size on the block search, which the library keeps for large ones."""
+    module = sys.modules["gpusparse.search"]
+    monkeypatch.setattr(module, "BLOCK_MIN_QUERIES", 1)
+    monkeypatch.setattr(module, "BLOCK_MIN_PAIRS", 1)
+
+
+def ref_of(csr):
+    return O.build_index(csr.indptr, csr.indices, csr.data, csr.shape[0], csr.shape[1])
+
+
+def check(ix, ref, ti, tw, k, what):
+    assert gs.search_plan(ix, ti.shape[0], ti.shape[1], k)["blocks"], what
+    print(f"blocks {what} B={ti.shape[0]} T={ti.shape[1]} k={k}", flush=True)
+    s, i = gs.search(ix, (ti, tw), k, path="fused")
+    es, _, ei = O.c_search(ref, ti, tw, k, threads=8)
+    assert np.array_equal(i.cpu().numpy(), ei), what
+    assert np.array_equal(s.cpu().numpy(), es), what
+
+
+def head_tail_csr(rng, n_docs, vocab, dtype, sign=False):
+    """Rows of a few of 300 frequent terms (more than the heavy ones) and of rare ones."""
+    rows = []
+    for _ in range(n_docs):
+        a = rng.choice(min(300, vocab), size=int(rng.integers(0, 20)), replace=False)
+        b = rng.choice(vocab, size=int(rng.integers(0, 12)), replace=False)
+        rows.append(np.unique(np.concatenate([a, b])))
+    indptr = np.concatenate([[0], np.cumsum([r.size for r in rows])]).astype(np.int64)
+    idx = np.concatenate(rows).astype(np.int32) if rows else np.zeros(0, np.int32)
+    w = rng.lognormal(-0.5, 0.8, size=idx.size)
+    if sign:
+        w *= rng.choice([-1.0, 1.0], size=idx.size, p=[0.3, 0.7])
+    return gs.CSR(indptr, idx, w.astype(dtype), (n_docs, vocab))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("sign", [False, True])
+def test_block_copy(device, dtype, sign):
+    """Levels and words decode to the weights within half a level; each block holds
+    its postings once."""
+    rng = np.random.default_rng(3)
+    n, V = 1000, 2000
+    csr = head_tail_csr(rng, n, V, dtype, sign)
+    ix = gs.build_from_csr(csr, device)
+    b = ensure_blocks(ix)
+    assert b.levels == (127 if sign else 255)
+    D = np.zeros((n, V))
+    D[np.repeat(np.arange(n), np.diff(csr.indptr)), csr.indices] = csr.data.astype(np.float64)
+    W = np.abs(D).max(axis=0)
+    heavy = b.heavy.cpu().numpy()
+    lengths = np.bincount(csr.indices, minlength=V)
+    assert np.array_equal(np.sort(lengths[heavy])[::-1], np.sort(lengths)[::-1][:H])
+    off = 128 if b.levels == 255 else 0
+    # bytes of a block: [doc / 16][term / 64][term % 64 / 16][doc % 16][term % 16]
+    lv = b.head.cpu().numpy().reshape(-1, 4, H // 64, 4, 16, 16).transpose(0, 1, 4, 2, 3, 5).reshape(-1, H)
+    lv = lv.astype(np.float64) + off
+    assert not lv[n:].any()
+    assert np.abs(lv[:n] * W[heavy] / b.levels - D[:, heavy]).max() <= 0.5003 * W[heavy].max() / b.levels
+    assert np.array_equal(lv[:n] != 0, np.rint(D[:, heavy] * (b.levels / W[heavy])) != 0)
+    rank, words, count = b.rank.cpu().numpy(), b.tail.cpu().numpy().view(np.uint32), b.count.cpu().numpy()
+    term_of = np.full(b.n_tail, -1)
+    tail_terms = np.flatnonzero(rank >= H)
+    term_of[rank[tail_terms] - H] = tail_terms
+    got = np.zeros((n, V))
+    held = np.zeros((n, V), dtype=int)
+    for blk in range(count.size):
+        w = words[csr.indptr[blk * 64]:][:count[blk]]
+        doc, t = blk * 64 + (w >> 16 & 63), term_of[w & 0xFFFF]
+        np.add.at(held, (doc, t), 1)
+        got[doc, t] = (w.view(np.int32) >> 22) * W[t] / 511
+    tail = np.setdiff1d(np.arange(V), heavy)
+    assert np.array_equal(held[:, tail], (D != 0)[:, tail].astype(int)) and not held[:, heavy].any()
+    assert (np.abs(got - D)[:, tail] <= 0.5003 * W[tail] / 511).all()
+
+
+@pytest.mark.parametrize("n_docs", [1, 63, 64, 65, 1000, 33000])
+@pytest.mark.parametrize("B", [1, 16, 65, 513])
+def test_block_edges(device, n_docs, B):
+    rng = np.random.default_rng(n_docs + B)
+    csr = head_tail_csr(rng, min(n_docs, 2000), 1500, np.float32)
+    if n_docs > 2000:  # repeat the rows: ties everywhere
+        m = -(-n_docs // 2000)
+        csr = gs.CSR(np.concatenate([[0], np.cumsum(np.tile(np.diff(csr.indptr), m))]).astype(np.int64),
+                     np.tile(csr.indices, m), np.tile(csr.data, m), (2000 * m, 1500))
+    ix = gs.build_from_csr(csr, device)
+    ref = ref_of(csr)
+    ti, tw = random_queries(rng, B, 1500, max_len=30, invalid_rate=0.05)
+    ti[B // 2:, ::2] %= 300
+    ti[0] = -1                                  # an empty query
+    for k in sorted({1, min(100, csr.shape[0]), min(1000, csr.shape[0])}):
+        check(ix, ref, ti, tw, k, f"n_docs={n_docs}")
+
+
+@pytest.mark.parametrize("kind", ["f16", "sign", "repeated", "query_signs", "tiny", "few_terms", "dup_tail", "unsorted",
+                                  "long_rows"])
+def test_block_weights(device, kind):
+    rng = np.random.default_rng(len(kind))
+    n, V = 5000, 3000
+    dt = np.float16 if kind == "f16" else np.float32
+    csr = head_tail_csr(rng, n, 40 if kind == "few_terms" else V, dt, kind == "sign")
+    if kind == "tiny":  # one heavy and some tail lists far below the others' weights
+        csr.data[csr.indices % 7 == 3] *= np.float32(1e-33)
+        csr.data[csr.indices % 7 == 4] *= np.float32(1e-6)
+    if kind == "dup_tail":  # a rare term twice in its docs
+        extra = np.zeros(n, dtype=int)
+        extra[::500] = 2
+        indptr = csr.indptr + np.concatenate([[0], np.cumsum(extra)])
+        idx, w = np.empty(indptr[-1], np.int32), np.empty(indptr[-1], np.float32)
+        for d in range(n):
+            a, b = csr.indptr[d], csr.indptr[d + 1]
+            row = np.concatenate([csr.indices[a:b], np.full(extra[d], V, np.int32)])
+            idx[indptr[d]:indptr[d + 1]] = row
+            w[indptr[d]:indptr[d + 1]] = np.concatenate([csr.data[a:b], np.arange(1, extra[d] + 1) * 0.37])
+        csr = gs.CSR(indptr.astype(np.int64), idx, w, (n, V + 1))
+    if kind == "unsorted":
+        for d in range(n):
+            p = rng.permutation(csr.indptr[d + 1] - csr.indptr[d]) + csr.indptr[d]
+            csr.indices[csr.indptr[d]:csr.indptr[d + 1]] = csr.indices[p]
+            csr.data[csr.indptr[d]:csr.indptr[d + 1]] = csr.data[p]
+    if kind == "long_rows":  # blocks of more postings than the copy's build stages in LDS
+        n = 200
+        m = 200 + 60 * (np.arange(n) % 2)
+        idx = np.concatenate([np.sort(rng.choice(V, size=x, replace=False)) for x in m]).astype(np.int32)
+        csr = gs.CSR(np.concatenate([[0], np.cumsum(m)]).astype(np.int64), idx,
+                     rng.lognormal(-0.5, 0.8, size=idx.size).astype(np.float32), (n, V))
+    ix = gs.build_from_csr(csr, device)
+    ref = ref_of(csr)
+    ti, tw = random_queries(rng, 70, csr.shape[1], max_len=30)
+    ti[:, :8] = rng.integers(0, min(300, csr.shape[1]), size=(70, 8))
+    tw[:, :8] = rng.lognormal(-0.5, 0.8, size=(70, 8))
+    if kind == "repeated":  # one heavy term up to 25 times, one of them large, and rare terms repeated
+        ti[:, 5:] = ti[:, 5:6]
+        tw[:, 6] = 3000.0
+        ti[35:, 20:] = 1700
+    if kind == "query_signs":
+        tw *= rng.choice([-1.0, 1.0], size=tw.shape, p=[0.4, 0.6]).astype(np.float32)
+    if kind == "dup_tail":
+        ti[::3, 9] = V
+        tw[::3, 9] = 2.0
+    for k in (10, min(500, n)):
+        check(ix, ref, ti, tw, k, kind)
+
+
+def test_block_fallback_rows(device):
+    """Rows the block search hands to the dense path: non-finite and huge query
+    weights, no positive score, fewer positive docs than k, candidates past the cap."""
+    rng = np.random.default_rng(8)
+    csr = head_tail_csr(rng, 3000, 900, np.float32)
+    ix = gs.build_from_csr(csr, device)
+    ref = ref_of(csr)
+    ti, tw = random_queries(rng, 60, 900, max_len=20)
+    tw[1] = 0.0
+    tw[2] *= -1.0
+    tw[3, 0] = 1e30
+    ti[4] = -1
+    ti[4, 0] = int(np.argmin(np.where(np.bincount(csr.indices, minlength=900) > 0,
+                                      np.bincount(csr.indices, minlength=900), 10 ** 9)))
+    check(ix, ref, ti, tw, 800, "fallback rows")
+    st = {}
+    s, i = gs.search(ix, (ti, tw), 50, path="fused", cand_cap=100, timing=st)
+    es, _, ei = O.c_search(ref, ti, tw, 50, threads=8)
+    assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(s.cpu().numpy(), es) and st["dense_rows"] > 0
+
+
+@pytest.mark.parametrize("cfg,n_docs,B,k", [("C2", 40000, 600, 1000), ("C3", 50001, 512, 1000), ("C4", 30000, 300, 1000),
+                                            ("C5", 40000, 200, 100)])
+def test_block_configs(device, cfg, n_docs, B, k):
+    docs, queries = synth.generate(synth.scaled(synth.CONFIGS[cfg], n_docs=n_docs, n_queries=B))
+    ix = gs.build_from_csr(docs, device)
+    ref = ref_of(docs)
+    ti, tw, _ = O.to_query_tensors(queries.indptr, queries.indices, queries.data)
+    if cfg == "C5":
+        tw = tw.astype(np.uint8)
+        s, i = gs.search(ix, (ti, tw), k, path="fused")
+        es, ei = O.search(ref, ti, tw, k)
+        assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(s.cpu().numpy(), es)
+        return
+    check(ix, ref, ti, tw, k, cfg)
+    cand, resc = gs.search_counts(ix, B, ti.shape[1], k)
+    assert (resc[cand >= k] >= k).all() and (cand >= resc).all()
