@@ -112,30 +112,76 @@ __global__ void k_term_count_global(const int32_t *__restrict__ idx, int64_t nnz
 }
 
 // padded = ceil32(lengths); offsets = exclusive scan(padded); optionally
-// delta = offsets - exclusive scan(lengths).  Single block of 1024 threads.
+// delta = offsets - exclusive scan(lengths).  Single block of 1024 threads: each of
+// its 16 waves sums its run of terms, then scans it 64 terms at a time from the
+// runs before, with two workgroup barriers in all (two scans with three barriers
+// each per 1024 terms took 66 us at V = 30522; now 50).
 __global__ void __launch_bounds__(1024) k_term_scan(const int32_t *lengths, int32_t V, int32_t *padded,
                                                     int64_t *offsets, int64_t *delta, int64_t *info,
                                                     const unsigned long long *n_bad) {
-    __shared__ int64_t sh[17];
-    __shared__ int64_t sh2[17];
-    int64_t carry = 0, carry_seg = 0;
-    for (int base = 0; base < V; base += blockDim.x) {
-        int i = base + threadIdx.x;
-        int64_t len = i < V ? lengths[i] : 0;
-        int64_t pad = (len + 31) & ~int64_t(31);
-        int64_t tot, tot2;
-        int64_t ex = block_excl_scan<int64_t>(pad, sh, &tot);
-        int64_t ex2 = block_excl_scan<int64_t>(len, sh2, &tot2);
-        if (i < V) {
-            if (padded) padded[i] = (int32_t)pad;
-            if (offsets) offsets[i] = carry + ex;
-            if (delta) delta[i] = (carry + ex) - (carry_seg + ex2);
+    constexpr int NW = 16, UN = 8;
+    __shared__ int64_t s_pad[NW], s_len[NW];
+    const int lane = gs_lane(), wave = gs_uniform((int)(threadIdx.x >> 6));
+    const int run = (((V + NW - 1) / NW) + 63) & ~63;
+    const int b = min(wave * run, V), e = min(b + run, V);
+    int64_t pad = 0, len = 0;
+    for (int i0 = b + lane; i0 < e; i0 += 64 * UN) {
+        int32_t l[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) l[u] = i0 + 64 * u < e ? lengths[i0 + 64 * u] : 0;
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            len += l[u];
+            pad += ((int64_t)l[u] + 31) & ~int64_t(31);
         }
-        carry += tot;
-        carry_seg += tot2;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        pad += __shfl_xor((long long)pad, d, 64);
+        len += __shfl_xor((long long)len, d, 64);
+    }
+    if (lane == 0) {
+        s_pad[wave] = pad;
+        s_len[wave] = len;
+    }
+    __syncthreads();
+    int64_t at_pad = 0, at_len = 0, total = 0;
+    for (int w = 0; w < NW; ++w) {
+        if (w < wave) {
+            at_pad += s_pad[w];
+            at_len += s_len[w];
+        }
+        total += s_pad[w];
+    }
+    for (int i0 = b; i0 < e; i0 += 64 * UN) {
+        int32_t l[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) l[u] = i0 + 64 * u + lane < e ? lengths[i0 + 64 * u + lane] : 0;
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            const int i = i0 + 64 * u + lane;
+            const int64_t p = ((int64_t)l[u] + 31) & ~int64_t(31);
+            int64_t xp = p, xl = l[u];
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int64_t op = __shfl_up((long long)xp, d, 64), ol = __shfl_up((long long)xl, d, 64);
+                if (lane >= d) {
+                    xp += op;
+                    xl += ol;
+                }
+            }
+            if (i < e) {
+                const int64_t off = at_pad + xp - p;
+                if (padded) padded[i] = (int32_t)p;
+                if (offsets) offsets[i] = off;
+                if (delta) delta[i] = off - (at_len + xl - l[u]);
+            }
+            at_pad += __shfl((long long)xp, 63, 64);
+            at_len += __shfl((long long)xl, 63, 64);
+        }
     }
     if (threadIdx.x == 0 && info) {
-        info[0] = carry;
+        info[0] = total;
         info[1] = n_bad ? (int64_t)*n_bad : 0;
     }
 }
@@ -549,7 +595,18 @@ __global__ void k_fill_pads(const int64_t *__restrict__ offsets, const int32_t *
 
 // ------------------------------------------------------------------ per-list scans
 
-constexpr int kListParts = 16;  // waves per list for the per-list passes
+constexpr int kListParts = 16;  // most waves per list for the per-list passes
+constexpr int64_t kListMaxBlocks = 0x7FFFFFFF;
+// Waves per list of a collection: one per 8192 docs.  Most lists are short, and a
+// launch of 16 waves for each of 30522 lists takes 150 us whatever they hold; a long
+// list's waves are latency-bound.  30K docs: list maxima 180 -> 37, order check 146
+// -> 33 us.  (The waves of all lists fit 32 bits.)
+inline int32_t list_parts(int64_t n_docs, int32_t vocab) {
+    int64_t p = n_docs / 8192;
+    p = p < 1 ? 1 : p > kListParts ? kListParts : p;
+    while (p > 1 && (int64_t)vocab * p >= ((int64_t)1 << 31)) --p;
+    return (int32_t)p;
+}
 constexpr int kListUnroll = 8;  // loads in flight per lane in those passes
 
 template <int WT>
@@ -562,15 +619,17 @@ __device__ __forceinline__ float weight_as_float(const void *w, int64_t i) {
 // max and max |w| per list, as monotone keys (max_key) and abs bits (max_abs_bits).
 template <int WT>
 __global__ void k_list_max(const void *__restrict__ w, const int64_t *__restrict__ offsets,
-                           const int32_t *__restrict__ lengths, int32_t V, uint32_t *max_key,
+                           const int32_t *__restrict__ lengths, int32_t V, int32_t parts, uint32_t *max_key,
                            uint32_t *max_abs_bits) {
     const int lane = gs_lane();
-    const int64_t wv = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-    const int64_t t = wv / kListParts;
-    const int part = (int)(wv % kListParts);
-    if (t >= V) return;
+    // a list's parts are neighbouring waves: the longest lists, the first terms in
+    // many vocabularies, start first whole
+    const uint32_t wv = (uint32_t)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
+    const uint32_t t = wv / (uint32_t)parts;
+    const int part = (int)(wv % (uint32_t)parts);
+    if (t >= (uint32_t)V) return;
     const int64_t L = lengths[t], o = offsets[t];
-    const int64_t per = (L + kListParts - 1) / kListParts;
+    const int64_t per = (L + parts - 1) / parts;
     const int64_t b = part * per, e = b + per < L ? b + per : L;
     if (b >= e) return;
     uint32_t mk = 0, ma = 0;
@@ -612,14 +671,16 @@ __global__ void k_list_max_final(const uint32_t *max_key, const uint32_t *max_ab
 
 // Non-ascending flag and count of equal neighbours per list.
 __global__ void k_check_lists(const int32_t *__restrict__ doc, const int64_t *__restrict__ offsets,
-                              const int32_t *__restrict__ lengths, int32_t V, int32_t *bad, int32_t *dup) {
+                              const int32_t *__restrict__ lengths, int32_t V, int32_t parts, int32_t *bad, int32_t *dup) {
     const int lane = gs_lane();
-    const int64_t wv = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
-    const int64_t t = wv / kListParts;
-    const int part = (int)(wv % kListParts);
-    if (t >= V) return;
+    // a list's parts are neighbouring waves: the longest lists, the first terms in
+    // many vocabularies, start first whole
+    const uint32_t wv = (uint32_t)((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6);
+    const uint32_t t = wv / (uint32_t)parts;
+    const int part = (int)(wv % (uint32_t)parts);
+    if (t >= (uint32_t)V) return;
     const int64_t L = lengths[t], o = offsets[t];
-    const int64_t per = (L + kListParts - 1) / kListParts;
+    const int64_t per = (L + parts - 1) / parts;
     int64_t b = part * per;
     const int64_t e = b + per < L ? b + per : L;
     if (b < 1) b = 1;
@@ -1303,8 +1364,9 @@ static int index_fill_impl(const int64_t *indptr_d, const int32_t *indices_d, co
     // max_scores / max_abs
     k_fill<uint32_t><<<gs_blocks(vocab, 256), 256, 0, s>>>(mk, vocab, 0u);
     k_fill<uint32_t><<<gs_blocks(vocab, 256), 256, 0, s>>>(ma, vocab, 0u);
-    k_list_max<WT><<<gs_blocks((int64_t)vocab * kListParts * 64, 256), 256, 0, s>>>(
-        weights_d, offsets_d, lengths_d, vocab, mk, ma);
+    const int32_t lparts = list_parts(n_docs, vocab);
+    k_list_max<WT><<<gs_blocks((int64_t)vocab * lparts * 64, 256, kListMaxBlocks), 256, 0, s>>>(
+        weights_d, offsets_d, lengths_d, vocab, lparts, mk, ma);
     k_list_max_final<<<gs_blocks(vocab, 256), 256, 0, s>>>(mk, ma, lengths_d, vocab, max_scores_d,
                                                           max_abs_d);
     GS_CHECK_LAUNCH();
@@ -1345,13 +1407,21 @@ extern "C" int gs_index_fill(const int64_t *indptr_d, const int32_t *indices_d, 
 
 extern "C" int gs_check_lists(const int32_t *doc_ids_d, const int64_t *offsets_d, const int32_t *lengths_d,
                               int32_t vocab, int32_t *bad_d, int32_t *dup_d, int64_t *info_d, void *stream) {
+    return gs_check_lists_sized(doc_ids_d, offsets_d, lengths_d, vocab, (int64_t)1 << 31, bad_d, dup_d, info_d, stream);
+}
+
+extern "C" int gs_check_lists_sized(const int32_t *doc_ids_d, const int64_t *offsets_d, const int32_t *lengths_d,
+                                    int32_t vocab, int64_t n_docs, int32_t *bad_d, int32_t *dup_d, int64_t *info_d,
+                                    void *stream) {
     GS_REQUIRE(vocab > 0, "vocab must be positive, got %d", vocab);
+    GS_REQUIRE(n_docs >= 0, "n_docs must not be negative");
     GS_REQUIRE(offsets_d && lengths_d && bad_d && dup_d && info_d, "null pointer");
     hipStream_t s = gs_stream(stream);
     k_fill<int32_t><<<gs_blocks(vocab, 256), 256, 0, s>>>(bad_d, vocab, 0);
     k_fill<int32_t><<<gs_blocks(vocab, 256), 256, 0, s>>>(dup_d, vocab, 0);
-    k_check_lists<<<gs_blocks((int64_t)vocab * kListParts * 64, 256), 256, 0, s>>>(
-        doc_ids_d, offsets_d, lengths_d, vocab, bad_d, dup_d);
+    const int32_t lparts = list_parts(n_docs, vocab);
+    k_check_lists<<<gs_blocks((int64_t)vocab * lparts * 64, 256, kListMaxBlocks), 256, 0, s>>>(
+        doc_ids_d, offsets_d, lengths_d, vocab, lparts, bad_d, dup_d);
     k_count_flags<<<1, 1024, 0, s>>>(bad_d, vocab, info_d);
     k_count_flags<<<1, 1024, 0, s>>>(lengths_d, vocab, info_d + 1);
     GS_CHECK_LAUNCH();
@@ -1367,11 +1437,12 @@ extern "C" int gs_list_max(const void *weights_d, int32_t wtype, const int64_t *
     hipStream_t s = gs_stream(stream);
     uint32_t *mk = reinterpret_cast<uint32_t *>(workspace_d), *ma = mk + vocab;
     k_fill<uint32_t><<<gs_blocks(2 * (int64_t)vocab, 256), 256, 0, s>>>(mk, 2 * (int64_t)vocab, 0u);
-    const unsigned g = gs_blocks((int64_t)vocab * kListParts * 64, 256);
+    const int32_t lparts = list_parts((int64_t)1 << 31, vocab);
+    const unsigned g = gs_blocks((int64_t)vocab * lparts * 64, 256, kListMaxBlocks);
     switch (wtype) {
-        case GS_W_F32: k_list_max<GS_W_F32><<<g, 256, 0, s>>>(weights_d, offsets_d, lengths_d, vocab, mk, ma); break;
-        case GS_W_F16: k_list_max<GS_W_F16><<<g, 256, 0, s>>>(weights_d, offsets_d, lengths_d, vocab, mk, ma); break;
-        case GS_W_U8: k_list_max<GS_W_U8><<<g, 256, 0, s>>>(weights_d, offsets_d, lengths_d, vocab, mk, ma); break;
+        case GS_W_F32: k_list_max<GS_W_F32><<<g, 256, 0, s>>>(weights_d, offsets_d, lengths_d, vocab, lparts, mk, ma); break;
+        case GS_W_F16: k_list_max<GS_W_F16><<<g, 256, 0, s>>>(weights_d, offsets_d, lengths_d, vocab, lparts, mk, ma); break;
+        case GS_W_U8: k_list_max<GS_W_U8><<<g, 256, 0, s>>>(weights_d, offsets_d, lengths_d, vocab, lparts, mk, ma); break;
         default: gs_set_error("unknown weight type %d", wtype); return GS_EINVAL;
     }
     k_list_max_final<<<gs_blocks(vocab, 256), 256, 0, s>>>(mk, ma, lengths_d, vocab, max_scores_d, max_abs_d);

@@ -146,6 +146,7 @@ SIGNATURES = {
                                 _P, _SZ, _P]),
     "gs_list_max": (C.c_int, [_P, _I32, _P, _P, _I32, _P, _P, _P, _SZ, _P]),
     "gs_check_lists": (C.c_int, [_P, _P, _P, _I32, _P, _P, _P, _P]),
+    "gs_check_lists_sized": (C.c_int, [_P, _P, _P, _I32, _I64, _P, _P, _P, _P]),
     "gs_chunk_bounds": (C.c_int, [_P, _P, _P, _I32, _I64, _I64, _P, _P]),
     "gs_tile_bounds": (C.c_int, [_P, _P, _P, _I32, _I64, _I32, _P, _P]),
     "gs_forward_fill_workspace": (_SZ, [_I64, _I32]),

@@ -296,9 +296,9 @@ def check_lists(index) -> tuple[int, int]:
     bad = torch.empty(V, dtype=torch.int32, device=dev)
     dup = torch.empty(V, dtype=torch.int32, device=dev)
     info = torch.zeros(2, dtype=torch.int64, device=dev)
-    _lib.check(L.gs_check_lists(_lib.ptr(index.doc_ids), _lib.ptr(index.offsets), _lib.ptr(index.lengths), V,
-                                _lib.ptr(bad), _lib.ptr(dup), _lib.ptr(info), _lib.stream_ptr(dev)),
-               "gs_check_lists")
+    _lib.check(L.gs_check_lists_sized(_lib.ptr(index.doc_ids), _lib.ptr(index.offsets), _lib.ptr(index.lengths), V,
+                                      int(index.num_docs), _lib.ptr(bad), _lib.ptr(dup), _lib.ptr(info),
+                                      _lib.stream_ptr(dev)), "gs_check_lists_sized")
     n_bad, n_nonempty = (int(x) for x in info.cpu())
     a = index.aux() if isinstance(index, GPUInvertedIndex) else {}
     a["n_bad_lists"] = n_bad

@@ -152,6 +152,11 @@ int gs_index_fill(const int64_t *indptr_d, const int32_t *indices_d, const void 
  */
 int gs_check_lists(const int32_t *doc_ids_d, const int64_t *offsets_d, const int32_t *lengths_d,
                    int32_t vocab, int32_t *bad_d, int32_t *dup_d, int64_t *info_d, void *stream);
+/* The same for an index of n_docs documents, which sets the launch shape (lists
+ * of any length are checked whatever it says). */
+int gs_check_lists_sized(const int32_t *doc_ids_d, const int64_t *offsets_d, const int32_t *lengths_d,
+                         int32_t vocab, int64_t n_docs, int32_t *bad_d, int32_t *dup_d, int64_t *info_d,
+                         void *stream);
 
 /* Per-list max weight (max_scores of run_correctness_verification.py:63,71: signed
  * max, 0 for empty lists) and max |weight|, for indexes assembled outside
