@@ -2,10 +2,10 @@
 
 Default workload (the headline metric): config C3 -- 8.8M synthetic docs
 (~1.06e9 postings, fp16 posting weights, fp32 accumulation), batches of 512
-queries, k = 1000.  A step is one ``search`` of one 512-query batch: the heavy
-terms' coarse sums (int8 matrix products), LDS-tile scoring of the other terms
-with threshold selection, candidate selection, fp64 rescoring and the status
-check.  Inputs (index and query batch) are resident in HBM before the timed
+queries, k = 1000.  A step is one ``search`` of one 512-query batch by the scorer
+that the library picks for it (at this size the block search: the rarer terms
+added in LDS tiles of 64 docs, the heavy ones as int8 matrix products on top, with
+threshold selection), candidate selection, fp64 rescoring and the status check.  Inputs (index and query batch) are resident in HBM before the timed
 region.
 
 Prints one JSON line.  ``value`` is queries/s with the results left in HBM (as
@@ -80,7 +80,8 @@ def parse():
     ap.add_argument("--path", default="fused", choices=["fused", "dense", "atomic"])
     ap.add_argument("--scorer", default="auto", choices=["auto", "hybrid", "lds"],
                     help="fused scorer: hybrid (heavy terms as int8 MFMA products, 16384-doc tiles), lds (LDS adds "
-                         "for every term) or auto (hybrid when the index allows it and no tile size is named)")
+                         "for every term) or auto (the library's choice: the block search for large batches, else "
+                         "hybrid, when the index allows it and no tile size is named)")
     ap.add_argument("--inflight", type=int, default=2,
                     help="batches in flight: batch i is queued before batch i - D's status is read (1: one at a time)")
     ap.add_argument("--streams", type=int, default=1,
@@ -280,6 +281,69 @@ def phase_matrix(timing):
     return np.array([[ev[i].elapsed_time(ev[i + 1]) for i in range(len(ev) - 1)] for ev in timing["phases"]])
 
 
+def scorer_args(a, hyb):
+    """Tile size and scorer a search is told: those named on the command line, else
+    none, so that the library picks (the block search for large batches)."""
+    return {"tile_log2": a.tile_log2, "hybrid": hyb} if a.named else {"tile_log2": None, "hybrid": None}
+
+
+def block_roofline(a, index, qt, k, plan, timing):
+    """Roofline of the block search's scoring launches (plan["blocks"]): every block
+    of 64 docs is read once per 512 queries -- the 128 heavy terms' int8 rows and one
+    4-byte word per posting of the other terms -- against the HBM peak; beside it the
+    int8 products (two limbs) and the LDS adds of the other terms' postings."""
+    import numpy as np
+
+    from gpusparse import _lib
+    from gpusparse.index import ensure_blocks
+    from gpusparse.search import search_index
+    sidx = search_index(index, plan["hybrid"])
+    b = ensure_blocks(sidx)
+    B, N, H = int(qt.shape[0]), int(index.num_docs), _lib.BLOCK_HEAVY
+    chunks = (B + 511) // 512
+    rows = int(b.count.numel()) * _lib.BLOCK_DOCS
+    words = int(b.count.sum().item())
+    nbytes = chunks * (rows * H + 4 * words)
+    avg_ms = float(np.mean([e0.elapsed_time(e1) for e0, e1 in timing["score_kernel"]]))
+    kern_ms = [e0.elapsed_time(e1) for e0, e1 in timing["score_kernel"]]
+    qt_h = qt.cpu().numpy()
+    valid = (qt_h >= 0) & (qt_h < index.vocab_size)
+    tq = np.where(valid, qt_h, 0)
+    length = index.lengths.cpu().numpy().astype(np.int64)
+    adds = int((length[tq] * (valid & (b.rank.cpu().numpy()[tq] >= H))).sum())
+    posts = int((length[tq] * valid).sum())
+    lds = lds_peak()
+    ops = 2 * 2 * H * rows * ((B + 15) // 16 * 16)
+    rate = adds / (avg_ms * 1e-3)
+    per_post = 4 + index.scores.element_size()
+    return {"bound": "hbm", "achieved": round(nbytes / (avg_ms * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
+            "frac": round(nbytes / (avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4), "traffic": None,
+            "bytes_per_launch": nbytes,
+            "bytes_note": f"algorithmic: {H} B of heavy-term levels per doc and 4 B per posting of the other terms, "
+                          "once per 512 queries; latency-bound (a block's chain of loads), not bandwidth-bound",
+            "lds_atomic": {"achieved": round(rate / 1e9, 1), "peak": None if lds is None else round(lds["peak"] / 1e9, 1),
+                           "unit": "G LDS atomic adds/s (one per scored posting of a term outside the products)",
+                           "frac": None if lds is None else round(rate / lds["peak"], 4)},
+            "mfma_int8": {"ops_per_launch": ops, "achieved": round(ops / (avg_ms * 1e-3) / 1e12, 1),
+                          "peak": PEAK_INT8_TOPS, "unit": "TOP/s",
+                          "frac": round(ops / (avg_ms * 1e-3) / 1e12 / PEAK_INT8_TOPS, 4)},
+            "hbm_physical": None,
+            "reference_stream_equiv": {
+                "bytes_per_launch": posts * per_post, "bytes_per_posting": per_post,
+                "GBs": round(posts * per_post / (avg_ms * 1e-3) / 1e9, 1),
+                "x_hbm_peak": round(posts * per_post / (avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 3),
+                "note": "the reference kernel's stream (each posting read once per (query, term): doc id + weight) "
+                        "over the scoring launches' time; here each posting is read once per 512 queries, so this is "
+                        "not a fraction of any hardware peak"},
+            "kernel": "k_blk_score (64-doc blocks: tail terms added in LDS, heavy terms as int8 products; all "
+                      "launches of a batch, with k_blk_deal and k_blk_tau between them)",
+            "kernel_ms_avg": round(avg_ms, 3), "kernel_ms_median": round(float(np.median(kern_ms)), 3),
+            "kernel_ms_min": round(float(np.min(kern_ms)), 3), "scored_postings_per_launch": adds,
+            "postings_in_launch_tiles": posts,
+            "search_call_ms_avg": round(float(np.mean([e0.elapsed_time(e1) for e0, e1 in timing["search"]])), 3),
+            "batch_scored_postings": posts}
+
+
 def time_search(a, index, qt, qw, k, hyb, depth, n_streams):
     """Times a.steps searches of one batch resident in HBM, with `depth` batches
     in flight over n_streams streams, after a.warmup untimed ones; then the same
@@ -293,9 +357,9 @@ def time_search(a, index, qt, qw, k, hyb, depth, n_streams):
     def step_async(timing=None):
         if a.path == "atomic":
             return gs.PendingSearch(gs.atomic_fused_score(index, qt, qw, k))
-        return gs.search_async(index, (qt, qw), k, tile_log2=a.tile_log2, path=a.path, unroll=a.unroll,
-                               waves=a.waves, tiles_per_wg=a.tiles_per_wg, sample_tiles=a.sample_tiles,
-                               timing=timing, hybrid=hyb)
+        return gs.search_async(index, (qt, qw), k, path=a.path, unroll=a.unroll, waves=a.waves,
+                               tiles_per_wg=a.tiles_per_wg, sample_tiles=a.sample_tiles, timing=timing,
+                               **scorer_args(a, hyb))
 
     # Batch i is queued on stream i mod S once batch i - D has finished (its
     # status read and any flagged rows completed), so up to D batches are in
@@ -379,8 +443,10 @@ def scorer_roofline(a, index, qt, T, k, hyb, timing, cfg_name):
     N = int(index.num_docs)
     n_tiles = (N + (1 << a.tile_log2) - 1) >> a.tile_log2
     # the main launch scores the tiles after the seed tiles
-    plan = gs.search_plan(index, B, T, k, tile_log2=a.tile_log2, sample_tiles=a.sample_tiles, unroll=a.unroll,
-                          tiles_per_wg=a.tiles_per_wg, hybrid=hyb)
+    plan = gs.search_plan(index, B, T, k, sample_tiles=a.sample_tiles, unroll=a.unroll,
+                          tiles_per_wg=a.tiles_per_wg, **scorer_args(a, hyb))
+    if plan["blocks"]:
+        return block_roofline(a, index, qt, k, plan, timing), plan, None
     S = min(plan["seed_tiles"], n_tiles)
     sidx = search_index(index, plan["hybrid"])  # a uint8 index's hybrid search runs on its float16 copy
     tb = sidx.aux()[("tile_bounds", a.tile_log2)]
@@ -594,7 +660,7 @@ def main():
     import gpusparse as gs
     from gpusparse import synth
     from gpusparse.index import ensure_search_state
-    from gpusparse.search import scorer_choice, search_index
+    from gpusparse.search import block_copy, scorer_choice, search_index
 
     if not torch.cuda.is_available():
         print("bench.py needs a GPU", file=sys.stderr)
@@ -623,10 +689,13 @@ def main():
         t_build = time.perf_counter() - t0
         t0 = time.perf_counter()
         tile, hyb = scorer_choice(ix, a.tile_log2 or None, want_hybrid)
-        ensure_search_state(search_index(ix, hyb), tile, hybrid=hyb)
+        sx = search_index(ix, hyb)
+        if a.named or block_copy(sx, a.batch or cfg.queries.n_rows, hyb, True) is None:
+            ensure_search_state(sx, tile, hybrid=hyb)
         torch.cuda.synchronize()
         return ix, ev, t_build, time.perf_counter() - t0, tile, hyb
 
+    a.named = bool(a.tile_log2 or a.scorer != "auto" or a.unroll or a.waves or a.tiles_per_wg or a.sample_tiles)
     want_hybrid = {"auto": None, "hybrid": True, "lds": False}[a.scorer]
     index, build_ev, t_build, t_state, a.tile_log2, hyb = build(docs)
     log(f"index built in {t_build:.2f}s (incl. H2D of the CSR); first-search state (tile bounds, packed copy, "
@@ -667,8 +736,8 @@ def main():
     # length) read, fp64 keys written and read back, the [B, k] results written.
     selection = None
     if a.path == "fused" and timing.get("phases"):
-        cand, resc = gs.search_counts(index, B, T, k, tile_log2=a.tile_log2, sample_tiles=a.sample_tiles,
-                                      unroll=a.unroll, tiles_per_wg=a.tiles_per_wg, hybrid=hyb)
+        cand, resc = gs.search_counts(index, B, T, k, sample_tiles=a.sample_tiles, unroll=a.unroll,
+                                      tiles_per_wg=a.tiles_per_wg, **scorer_args(a, hyb))
         per = phase_matrix(timing)
         sel_ms = float(np.median(per[:, 4:7].sum(axis=1)))
         n_cand = int(np.minimum(cand.astype(np.int64), plan["cand_cap"] if plan else 65536).sum())
@@ -772,7 +841,7 @@ def main():
                    "path": a.path, "inflight": max(1, a.inflight, a.streams), "streams": a.streams,
                    "scorer": None if plan is None else {key: plan[key] for key in
                                                         ("group_size", "unroll", "tiles_per_wg", "seed_tiles", "packed",
-                                                         "hybrid")}},
+                                                         "hybrid", "blocks")}},
         "ms_per_batch_one_in_flight": None if one_ms is None else round(one_ms, 3),
         "roofline": roof, "heavy_terms_kernel": head, "selection": selection, "index_build": index_build,
         "cpu_baseline": cpu, "parity": parity, "components_ms": components,
