@@ -515,7 +515,7 @@ def ensure_blocks(index) -> Blocks | None:
         if a.get("fwd") is None:
             a["fwd"] = build_forward(index)
         ptr, terms, w = a["fwd"]
-        order = a.pop("block_order")
+        order = a["block_order"]
         rank = np.full(V, -1, dtype=np.int32)
         rank[order] = np.arange(order.size, dtype=np.int32)
         heavy = np.full(_lib.BLOCK_HEAVY, -1, dtype=np.int32)
