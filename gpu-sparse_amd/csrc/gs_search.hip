@@ -856,6 +856,11 @@ constexpr int kUnionThreads = 512;  // 8 waves; two workgroups per CU
 constexpr int kUnionBatch = 220;    // union terms described in LDS at a time
 constexpr int kEmitChunks = (int)(kUnionTileLds / 4 / 256);  // 256-doc emission chunks of one workgroup
 constexpr int kLocalBins = 256;  // bins of the per-slot score histogram of the seed launch
+// Fewest results for which the seed launch counts its candidates in LDS first: at
+// 1000 (16 queries on 8.8M docs) the batch takes 649 instead of 715 us, the device
+// atomics of a tile's best docs queueing up at a few bins; at 100 and 10 the
+// window's clearing and hand-over cost as much (617 / 613, 184 / 179 us).
+constexpr int kLocalCountK = 256;
 constexpr int kLocalSlots = 4;   // slots per workgroup that get a local threshold
 constexpr int kEmitReads = 4;    // emission chunks a wave reads at once in the counting pass
 
@@ -864,6 +869,10 @@ constexpr size_t kUnionMetaLds =
     (size_t)kUnionBatch * 8 + (size_t)kUnionBatch * 4 + (size_t)(kUnionBatch + 2) * 8 + (size_t)kUnionBatch * 12;
 static_assert(kUnionTileLds + kUnionMetaLds + kStaticLdsBudget <= kLdsPerWg / 2,
               "two scoring workgroups must fit the 160 KiB of LDS of a CU");
+
+// Right shift of the seed launch's local bins: a slot's maximum score lands below kLocalBins.
+__device__ __forceinline__ int local_shift(uint32_t top) { return max(24 - __clz((int)(top | 1u)), 0); }
+static_assert(kLocalBins == 256, "local_shift");
 
 // ---------------------------------------------------------------------- candidate emission
 
@@ -883,11 +892,20 @@ struct EmitArgs {
 // Pass 1 counts each chunk's candidates; one wave per slot scans the slot's
 // chunk counts (one per lane) and reserves the slot's range with one global
 // atomic; pass 2 revisits only the chunks holding candidates (a wave reads its
-// chunk counts at once, one per lane).  Whole workgroup (kUnionThreads) calls it.
+// chunk counts at once, one per lane).  With `local` (the seed launch, whose
+// candidates are a tile's k best and fall into few bins) a slot's candidates are
+// counted in `lhist`, in the window of histogram bins that ends at its maximum's,
+// and go to the query's histogram with one atomic per bin; those below the window
+// go there one by one.  (Every candidate of the main launch, too: slower, it has a
+// dozen per slot and tile.)  Whole workgroup (kUnionThreads) calls it.
 __device__ __forceinline__ void emit_slices(const EmitArgs &a, const uint32_t *acc, int nq, int cps_log2,
                                             int64_t doc0, int grp, uint32_t *s_thr, uint32_t *s_off,
-                                            uint32_t *s_ccnt, uint32_t *s_base, uint32_t *s_emit, uint32_t *s_maxb) {
+                                            uint32_t *s_ccnt, uint32_t *s_base, uint32_t *s_emit, uint32_t *s_maxb,
+                                            bool local, uint32_t *lhist, const int32_t *s_wbin) {
     constexpr int NW = kUnionThreads / 64;
+    const int wlog2 = nq == 1 ? 10 : 8;  // bins of a slot's window in lhist
+    if (local)
+        for (int i = threadIdx.x; i < kLocalSlots * kLocalBins; i += kUnionThreads) lhist[i] = 0;
     const int tid = threadIdx.x, lane = gs_lane();
     const int wave = gs_uniform(tid >> 6);
     const int cps = 1 << cps_log2;
@@ -974,7 +992,9 @@ __device__ __forceinline__ void emit_slices(const EmitArgs &a, const uint32_t *a
                     a.cand_key[(int64_t)q * a.cap + slot] = vv[u];
                 }
                 const uint32_t b = gs_bin_of((float)vv[u]);
-                atomicAdd(a.hist + (int64_t)q * GS_HIST_BINS + b, 1u);
+                const int wb = local ? (int)b - s_wbin[g] : -1;
+                if (wb >= 0) atomicAdd(lhist + (g << wlog2) + wb, 1u);
+                else atomicAdd(a.hist + (int64_t)q * GS_HIST_BINS + b, 1u);
                 mb = b > mb ? b : mb;
             }
             base += (uint32_t)__popcll(mk[u]);
@@ -982,6 +1002,15 @@ __device__ __forceinline__ void emit_slices(const EmitArgs &a, const uint32_t *a
         if (mb) atomicMax(&s_maxb[g], mb);  // lanes holding candidates
     }
     __syncthreads();
+    if (local) {
+        for (int i = tid; i < (nq << wlog2); i += kUnionThreads) {
+            const int g = i >> wlog2;
+            if (lhist[i])
+                atomicAdd(a.hist + (int64_t)(grp * a.G + g) * GS_HIST_BINS + s_wbin[g] + (i & ((1 << wlog2) - 1)),
+                          lhist[i]);
+        }
+        __syncthreads();
+    }
     // tau is recomputed from the histogram when a slot's candidate count crosses
     // a multiple of max(k / 8, 64) at or above k; otherwise only the max bin is
     // published
@@ -1028,6 +1057,8 @@ __global__ void __launch_bounds__(kUnionThreads, HD ? 4 : 2) k_score_union(const
     __shared__ int32_t s_scan[kUnionThreads / 64 + 1];
     __shared__ uint32_t s_thr[32], s_emit[32], s_maxb[32], s_base[32], s_mfix[32];
     __shared__ uint32_t s_lhist[kLocalSlots][kLocalBins];
+    __shared__ int32_t s_wbin[kLocalSlots];
+    static_assert(kLocalSlots * kLocalBins == 1024, "a single slot's window");
     __shared__ uint32_t s_off[kEmitChunks], s_ccnt[kEmitChunks];
 
     const int tid = threadIdx.x, lane = gs_lane();
@@ -1457,12 +1488,17 @@ __global__ void __launch_bounds__(kUnionThreads, HD ? 4 : 2) k_score_union(const
     const int cps_log2 = a.tile_log2 - 8;  // 256-doc chunks per slice = 1 << cps_log2
     const int nce = nq << cps_log2;        // <= kEmitChunks (G * TILE <= kUnionTileLds / 4)
     if (tid < nq) s_thr[tid] = emit_threshold(r_tau, s_mfix[tid]);
-    if (a.local_k > 0 && nq <= kLocalSlots) {
+    const bool seed = a.local_k > 0 && nq <= kLocalSlots;
+    if (seed) {
         // Seed launch (tau = 0): every positive doc would be a candidate.  Any k
         // docs of this tile scoring >= X bound the query's k-th score from below
         // by X, so the slot's local k-th score L gives the threshold L - margin.
-        // L is bounded from below by the lower edge of the histogram bin (linear
-        // over (0, slot max]) where the count from the top reaches k.
+        // L is bounded from below by the lower edge of the histogram bin where the
+        // count from the top reaches k.  Bins are the score shifted right until the
+        // slot's maximum is below 256: a division by the maximum per doc made up much of
+        // the launch (200 queries on 300K docs: 62 -> 45 us).  Bin 0 is not counted: its
+        // docs, often most of the tile, would queue up at one address, and its edge
+        // bounds nothing.
         if (tid < nq) s_maxb[tid] = 0;
         for (int i = tid; i < kLocalSlots * kLocalBins; i += kUnionThreads) (&s_lhist[0][0])[i] = 0;
         __syncthreads();
@@ -1475,12 +1511,14 @@ __global__ void __launch_bounds__(kUnionThreads, HD ? 4 : 2) k_score_union(const
         __syncthreads();
         for (int ch = wave; ch < nce; ch += NW) {
             const int g = ch >> cps_log2;
-            const uint64_t span = (uint64_t)s_maxb[g] + 1;
+            const int sh = local_shift(s_maxb[g]);
             const uint4 v4 = *reinterpret_cast<const uint4 *>(acc + ((size_t)ch << 8) + 4 * lane);
             const uint32_t vs[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if ((int32_t)vs[u] > 0) atomicAdd(&s_lhist[g][(uint64_t)vs[u] * kLocalBins / span], 1u);
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t b = (int32_t)vs[u] > 0 ? vs[u] >> sh : 0u;
+                if (b) atomicAdd(&s_lhist[g][b], 1u);
+            }
         }
         __syncthreads();
         for (int g = wave; g < nq; g += NW) {  // lane l: bins 255 - 4l .. 252 - 4l
@@ -1495,20 +1533,25 @@ __global__ void __launch_bounds__(kUnionThreads, HD ? 4 : 2) k_score_union(const
                     uint32_t cum = inc - sum;
                     int j = 0;
                     while (cum + c[j] < (uint32_t)a.local_k) cum += c[j++];
-                    const uint64_t b = (uint64_t)(kLocalBins - 1 - 4 * lane - j);
-                    const uint64_t span = (uint64_t)s_maxb[g] + 1;
-                    const uint32_t edge = (uint32_t)((b * span + kLocalBins - 1) / kLocalBins);  // least v of bin b
+                    const uint32_t b = (uint32_t)(kLocalBins - 1 - 4 * lane - j);
+                    const uint32_t edge = b << local_shift(s_maxb[g]);  // least v of bin b
                     const uint32_t t = emit_threshold(edge, s_mfix[g]);
                     if (t > s_thr[g]) s_thr[g] = t;
                 }
             }
         }
         __syncthreads();
-        if (tid < nq) s_maxb[tid] = 0;
+        if (tid < nq) {
+            // the first bin of the slot's window in s_lhist: the window ends at the
+            // maximum's bin, and starts at bin 0 at the earliest
+            s_wbin[tid] = max((int)gs_bin_of((float)s_maxb[tid]) - ((nq == 1 ? 1024 : kLocalBins) - 1), 0);
+            s_maxb[tid] = 0;
+        }
     }
     __syncthreads();
     const EmitArgs ea{a.tau, a.cnt, a.maxbin, a.hist, a.cand_doc, a.cand_key, a.G, a.cap, a.k};
-    emit_slices(ea, acc, nq, cps_log2, doc0, grp, s_thr, s_off, s_ccnt, s_base, s_emit, s_maxb);
+    emit_slices(ea, acc, nq, cps_log2, doc0, grp, s_thr, s_off, s_ccnt, s_base, s_emit, s_maxb,
+                seed && a.local_k >= kLocalCountK, &s_lhist[0][0], s_wbin);
     }  // tile
 }
 

@@ -274,6 +274,27 @@ def test_hybrid_launch_shapes_and_dirty_workspace(device, tile_log2, tiles_per_w
     check(ix, ref, ti, tw, 60, **kw)
 
 
+@pytest.mark.parametrize("spread", [0, 14])
+@pytest.mark.parametrize("tile_log2", [12, 13, 14])
+@pytest.mark.parametrize("k", [255, 256, 1000, 3000])
+def test_seed_candidates_counted_in_lds(device, spread, tile_log2, k):
+    """The seed launch at the k from which it counts its candidates in LDS, groups of
+    1, 2 and 4 queries a workgroup (5 queries: a short last group), scores within one octave (a single run of bins) and over 14 octaves
+    (candidates below the window go to the histogram one by one), hybrid and not."""
+    rng = np.random.default_rng(spread + k)
+    csr = zipf_csr(rng, 24000, 300, np.float32, max_len=6)
+    csr.data[:] = np.exp2(-spread * rng.random(csr.data.size)).astype(np.float32)
+    ix = gs.build_from_csr(csr, device)
+    ref = oracle_index(csr)
+    ti, tw = zipf_queries(rng, 5, 300, np.float32, max_len=6)
+    ti[1] = -1  # no terms: every score is 0
+    print(f"seed candidates spread={spread} tile_log2={tile_log2} k={k}", flush=True)
+    check(ix, ref, ti, tw, k, tile_log2=tile_log2)
+    s, i = gs.search(ix, (torch.from_numpy(ti), torch.from_numpy(tw)), k, path="fused", hybrid=False)
+    vs, _, vi = O.c_search(ref, ti, tw, k, threads=8)
+    assert np.array_equal(i.cpu().numpy(), vi) and np.array_equal(s.cpu().numpy(), vs)
+
+
 def test_hybrid_not_used_when_heavy_lists_repeat_docs(device):
     """An index whose heavy lists repeat a doc cannot hold a single dense cell
     per (doc, heavy term): hybrid=True raises and the default search runs the
