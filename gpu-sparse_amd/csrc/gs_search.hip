@@ -3088,6 +3088,7 @@ extern "C" int gs_search_blocks_workspace(const gs_index *index, const gs_block_
                                           int32_t k, const gs_search_opts *opts, size_t *bytes) {
     if (int rc = check_blocks(index, blocks)) return rc;
     GS_REQUIRE(B > 0 && T > 0 && k > 0 && bytes, "bad search sizes");
+    GS_REQUIRE(T <= kGroupSortCap, "query width T=%d exceeds %d terms", T, kGroupSortCap);
     gs_arena ar{nullptr, 0, 0};
     plan_blocks(index, blocks, B, T, k, opts, ar);
     *bytes = ar.used + 256;
@@ -3101,6 +3102,8 @@ extern "C" int gs_search_blocks(const gs_index *index, const gs_block_copy *bloc
     if (int rc = check_blocks(index, blocks)) return rc;
     GS_REQUIRE(B > 0 && T > 0, "empty query batch (B=%d, T=%d)", B, T);
     GS_REQUIRE(k >= 1 && k <= kMaxK && (int64_t)k <= index->n_docs, "k=%d outside [1, min(n_docs, %d)]", k, kMaxK);
+    // (a chunk's entries, kBlkMaxQ T words, then stay far below the 4 GiB of a buffer resource)
+    GS_REQUIRE(T <= kGroupSortCap, "query width T=%d exceeds %d terms", T, kGroupSortCap);
     GS_REQUIRE((int64_t)B * T < (1ll << 31), "query batch too large (B=%d, T=%d)", B, T);
     GS_REQUIRE(q_terms_d && q_weights_d && out_scores_d && out_ids_d && status_d && workspace_d, "null pointer");
     hipStream_t s = gs_stream(stream);
@@ -3116,6 +3119,7 @@ extern "C" int gs_search_blocks_counts(const gs_index *index, const gs_block_cop
                                        uint32_t *cand_d, uint32_t *resc_d, void *stream) {
     if (int rc = check_blocks(index, blocks)) return rc;
     GS_REQUIRE(B > 0 && T > 0 && k > 0 && workspace_d && cand_d && resc_d, "bad arguments");
+    GS_REQUIRE(T <= kGroupSortCap, "query width T=%d exceeds %d terms", T, kGroupSortCap);
     gs_arena ar{reinterpret_cast<char *>(const_cast<void *>(workspace_d)), 0, workspace_bytes};
     const BlkPlan p = plan_blocks(index, blocks, B, T, k, opts, ar);
     GS_REQUIRE(ar.ok(), "workspace smaller than the search's (%zu < %zu bytes)", workspace_bytes, ar.used);

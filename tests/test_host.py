@@ -51,6 +51,32 @@ def test_argument_errors_map_to_python_exceptions():
         _lib.check(rc, "gs_head_fill")
 
 
+def test_block_search_refuses_wide_queries():
+    """The three block-search calls take the query widths gs_search takes: a chunk's
+    entry array must stay within one 32-bit buffer resource.  Rejected on the host,
+    before any pointer is used."""
+    L = _lib.lib()
+    idx, blk = _lib.GsIndex(), _lib.GsBlockCopy()
+    idx.n_docs, idx.vocab, idx.wtype = 1000, 100, _lib.GS_W_F32
+    for f in ("max_abs_d", "dup_d", "fwd_ptr_d", "fwd_terms_d", "fwd_weights_d"):
+        setattr(idx, f, 8)
+    for f in ("head_d", "tail_d", "count_d", "rank_d", "heavy_d"):
+        setattr(blk, f, 8)
+    blk.n_tail, blk.levels = 50, 255
+    ix, bk, P = ctypes.byref(idx), ctypes.byref(blk), ctypes.c_void_p(8)
+    need = ctypes.c_size_t()
+    assert L.gs_search_blocks_workspace(ix, bk, 16, 8192, 10, None, ctypes.byref(need)) == _lib.GS_OK
+    for T in (8193, 1 << 26):
+        calls = {
+            "gs_search_blocks_workspace": L.gs_search_blocks_workspace(ix, bk, 16, T, 10, None, ctypes.byref(need)),
+            "gs_search_blocks": L.gs_search_blocks(ix, bk, P, P, 16, T, 10, None, P, P, P, P, 0, None),
+            "gs_search_blocks_counts": L.gs_search_blocks_counts(ix, bk, 16, T, 10, None, P, 0, P, P, None),
+        }
+        for name, rc in calls.items():
+            with pytest.raises(ValueError, match=f"query width T={T} exceeds 8192"):
+                _lib.check(rc, name)
+
+
 def test_pack_shift_matches_oracle():
     """gs_pack_shift is host code: the C ABI and the oracle agree on random,
     power-of-two and extreme magnitudes, and reject negative / non-finite input."""
