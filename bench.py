@@ -740,7 +740,7 @@ def main():
                                       tiles_per_wg=a.tiles_per_wg, **scorer_args(a, hyb))
         per = phase_matrix(timing)
         sel_ms = float(np.median(per[:, 4:7].sum(axis=1)))
-        n_cand = int(np.minimum(cand.astype(np.int64), plan["cand_cap"] if plan else 65536).sum())
+        n_cand = int(np.minimum(cand.astype(np.int64), (plan and plan["cand_cap"]) or 65536).sum())
         n_resc = int(resc.astype(np.int64).sum())
         row_bytes = 16 + (int(index.lengths.sum().item()) / max(1, int(index.num_docs))) * (4 + wbytes)
         sel_bytes = n_cand * 8 + n_resc * 4 + int(n_resc * row_bytes) + n_resc * 8 + n_resc * 12 + B * k * 12

@@ -170,13 +170,14 @@ def _opts(sample_tiles=0, cand_cap=0, unroll=0, waves=0, tiles_per_wg=0, batch_o
 WORKSPACE_STREAMS = 4  # streams whose fused-search workspaces an index keeps
 
 
-def _workspace(index, nbytes: int, stream_key: int = 0) -> torch.Tensor:
+def _workspace(index, nbytes: int, stream_key: int = 0, plan=None) -> torch.Tensor:
     """The index's fused-search workspace for one stream (searches in flight on
     different streams must not share one; on one stream they run in order).  The
     index keeps those of its WORKSPACE_STREAMS most recently used streams (a
     dropped one is freed once the searches queued with it are done: the
     allocator orders its reuse on its stream).  The one last handed out is also
-    aux()["workspace"], which search_counts reads."""
+    aux()["workspace"], which search_counts reads, and its `plan` (_plan_key)
+    aux()["workspace_plan"]."""
     a = index.aux()
     pool = a.setdefault("workspaces", OrderedDict())
     ws = pool.get(stream_key)
@@ -187,8 +188,21 @@ def _workspace(index, nbytes: int, stream_key: int = 0) -> torch.Tensor:
     pool.move_to_end(stream_key)
     while len(pool) > WORKSPACE_STREAMS:
         pool.popitem(last=False)
-    a["workspace"] = ws
+    a["workspace"], a["workspace_plan"] = ws, plan
     return ws
+
+
+def _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch_order) -> bool:
+    """Whether a call names neither a scorer nor a launch shape (`waves` is none:
+    gs_search ignores it), so that large batches take the block search."""
+    return hybrid is None and tile_log2 is None and not (sample_tiles or unroll or tiles_per_wg or batch_order)
+
+
+def _plan_key(blocks: bool, B, T, kk, cand_cap, *scorer_args) -> tuple:
+    """What lays a fused search's workspace out: the arrays of gs_search_blocks
+    follow from the first arguments, those of gs_search from the scorer's too."""
+    return ("blocks" if blocks else "scorer", int(B), int(T), int(kk), int(cand_cap)) + \
+        (() if blocks else tuple(int(x) for x in scorer_args))
 
 
 def _dense_rows(index, gidx, qt, qw, k, rows, out_s, out_i, dense_budget):
@@ -344,8 +358,7 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
         qt = torch.full((B, 1), -1, dtype=torch.int32, device=dev)
         qw = torch.zeros((B, 1), dtype=qw.dtype, device=dev)
         T = 1
-    default_scorer = hybrid is None and tile_log2 is None and not (sample_tiles or unroll or waves or tiles_per_wg or
-                                                                   batch_order)
+    default_scorer = _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch_order)
     tile_arg, hybrid_arg = tile_log2, hybrid
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     if path not in ("auto", "fused", "dense"):
@@ -399,7 +412,9 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
     else:
         gidx = gs_index_struct(index, tile_log2, hyb)
         _lib.check(L.gs_search_workspace(ref(gidx), B, T, kk, ref(opts), ref(need)), "gs_search_workspace")
-    ws = _workspace(index, int(need.value), stream.cuda_stream)
+    ws = _workspace(index, int(need.value), stream.cuda_stream,
+                    _plan_key(blocks is not None, B, T, kk, cand_cap, tile_log2, hyb, sample_tiles, unroll,
+                              tiles_per_wg, batch_order))
     status = torch.empty(B, dtype=torch.int32, device=dev)
     s = _lib.stream_ptr(dev)
     if timing is not None:
@@ -478,12 +493,14 @@ def search_plan(index, B: int, T: int, k: int, *, tile_log2: int | None = None, 
     """How the fused path of `search` runs a batch of B queries of width T
     (gs_search_plan): seed tiles, queries per group, postings per lane per chunk,
     tiles per scoring workgroup, whether the packed copy is read and whether the
-    hybrid scorer runs; "blocks": whether the block search runs in its place (the
-    other entries then say what the hybrid scorer would do)."""
-    default_scorer = hybrid is None and tile_log2 is None and not (sample_tiles or unroll or tiles_per_wg or batch_order)
+    hybrid scorer runs; "blocks": whether the block search runs in its place (those
+    entries are then None: the scorer's own copies are not made for such batches)."""
+    default_scorer = _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch_order)
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     index = search_index(index, hyb)
-    blocks = block_copy(index, int(B), hyb, default_scorer)
+    if block_copy(index, int(B), hyb, default_scorer) is not None:
+        return {"tile_log2": tile_log2, "seed_tiles": None, "group_size": None, "unroll": None, "tiles_per_wg": None,
+                "packed": None, "hybrid": hyb, "cand_cap": None, "blocks": True}
     gidx = gs_index_struct(index, tile_log2, hyb)
     opts = _opts(sample_tiles, cand_cap, unroll, 0, tiles_per_wg, batch_order, hyb)
     info = _lib.GsSearchPlanInfo()
@@ -491,38 +508,38 @@ def search_plan(index, B: int, T: int, k: int, *, tile_log2: int | None = None, 
                                          _lib.C.byref(opts), _lib.C.byref(info)), "gs_search_plan")
     return {"tile_log2": tile_log2, "seed_tiles": info.seed_tiles, "group_size": info.group_size,
             "unroll": info.unroll, "tiles_per_wg": info.tiles_per_wg, "packed": bool(info.packed),
-            "hybrid": bool(info.hybrid), "cand_cap": info.cand_cap, "blocks": blocks is not None}
+            "hybrid": bool(info.hybrid), "cand_cap": info.cand_cap, "blocks": False}
 
 
 def search_counts(index, B: int, T: int, k: int, *, tile_log2: int | None = None, sample_tiles: int = 0,
                   cand_cap: int = 0, unroll: int = 0, tiles_per_wg: int = 0, batch_order: bool = False,
                   hybrid: bool | None = None):
-    """Per scoring slot of the fused search that last ran with these arguments:
-    (docs the scorer emitted as candidates, candidates rescored in fp64), two
-    numpy uint32 [B] arrays (gs_search_counts on the index's cached workspace)."""
-    default_scorer = hybrid is None and tile_log2 is None and not (sample_tiles or unroll or tiles_per_wg or batch_order)
+    """Per scoring slot of the fused search that last ran, with these arguments (ValueError
+    when it ran with others): (docs the scorer emitted as candidates, candidates
+    rescored in fp64), two numpy uint32 [B] arrays (gs_search_counts or
+    gs_search_blocks_counts on the index's cached workspace)."""
+    default_scorer = _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch_order)
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     index = search_index(index, hyb)
-    ws = index.aux().get("workspace")
+    ws, plan = index.aux().get("workspace"), index.aux().get("workspace_plan")
     if ws is None:
         raise ValueError("no fused search has run on this index")
     dev = _device_of(index)
-    opts = _opts(sample_tiles, cand_cap, unroll, 0, tiles_per_wg, batch_order, hyb)
+    kk = min(int(k), int(index.num_docs))
     blocks = block_copy(index, int(B), hyb, default_scorer)
+    if plan != _plan_key(blocks is not None, B, T, kk, cand_cap, tile_log2, hyb, sample_tiles, unroll, tiles_per_wg,
+                         batch_order):
+        raise ValueError(f"the last fused search on this index ran with other arguments: {plan}")
+    opts = _opts(sample_tiles, cand_cap, unroll, 0, tiles_per_wg, batch_order, hyb)
+    ref, ptr, L = _lib.C.byref, _lib.ptr, _lib.lib()
+    cand, resc = (torch.empty(B, dtype=torch.int32, device=dev) for _ in range(2))
+    tail = (int(B), int(T), kk, ref(opts), ptr(ws), ws.numel(), ptr(cand), ptr(resc), _lib.stream_ptr(dev))
     if blocks is not None:
         gidx, bcopy = gs_blocks_index(index), blocks.struct()
-        cand, resc = (torch.empty(B, dtype=torch.int32, device=dev) for _ in range(2))
-        _lib.check(_lib.lib().gs_search_blocks_counts(_lib.C.byref(gidx), _lib.C.byref(bcopy), int(B), int(T),
-                                                      min(int(k), int(index.num_docs)), _lib.C.byref(opts),
-                                                      _lib.ptr(ws), ws.numel(), _lib.ptr(cand), _lib.ptr(resc),
-                                                      _lib.stream_ptr(dev)), "gs_search_blocks_counts")
-        return cand.cpu().numpy().view(np.uint32), resc.cpu().numpy().view(np.uint32)
-    gidx = gs_index_struct(index, tile_log2, hyb)
-    cand = torch.empty(B, dtype=torch.int32, device=dev)
-    resc = torch.empty(B, dtype=torch.int32, device=dev)
-    _lib.check(_lib.lib().gs_search_counts(_lib.C.byref(gidx), int(B), int(T), min(int(k), int(index.num_docs)),
-                                           _lib.C.byref(opts), _lib.ptr(ws), ws.numel(), _lib.ptr(cand),
-                                           _lib.ptr(resc), _lib.stream_ptr(dev)), "gs_search_counts")
+        _lib.check(L.gs_search_blocks_counts(ref(gidx), ref(bcopy), *tail), "gs_search_blocks_counts")
+    else:
+        gidx = gs_index_struct(index, tile_log2, hyb)
+        _lib.check(L.gs_search_counts(ref(gidx), *tail), "gs_search_counts")
     return cand.cpu().numpy().view(np.uint32), resc.cpu().numpy().view(np.uint32)
 
 

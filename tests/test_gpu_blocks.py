@@ -198,3 +198,33 @@ def test_block_configs(device, cfg, n_docs, B, k):
     check(ix, ref, ti, tw, k, cfg)
     cand, resc = gs.search_counts(ix, B, ti.shape[1], k)
     assert (resc[cand >= k] >= k).all() and (cand >= resc).all()
+
+
+def test_block_counts_and_plan(device):
+    """search_counts reads the workspace as the search that last used it laid it out:
+    `waves`, which names no launch shape, keeps the block search, and counts of
+    another search are refused.  A plan that answers "blocks" makes none of the
+    other scorer's copies."""
+    rng = np.random.default_rng(21)
+    csr = head_tail_csr(rng, 4000, 1500, np.float32)
+    ix = gs.build_from_csr(csr, device)
+    ti, tw = random_queries(rng, 40, 1500, max_len=20)
+    ti[:, 0], tw[:, 0] = 7, 1.0
+    B, T, k = 40, ti.shape[1], 50
+    plan = gs.search_plan(ix, B, T, k)
+    assert plan["blocks"] and "head" not in ix.aux() and \
+        not any(isinstance(key, tuple) and key[0] == "packed" for key in ix.aux())
+    gs.search(ix, (ti, tw), k, path="fused", waves=8)
+    cand, resc = gs.search_counts(ix, B, T, k)
+    gs.search(ix, (ti, tw), k, path="fused")
+    cand2, resc2 = gs.search_counts(ix, B, T, k)
+    assert np.array_equal(cand, cand2) and np.array_equal(resc, resc2)
+    assert (cand >= resc).all() and (cand <= 4000).all() and (cand >= k).all()
+    for args, opts in (((B, T, k + 1), {}), ((B, T, k), {"hybrid": True}), ((B, T, k), {"cand_cap": 4096})):
+        with pytest.raises(ValueError, match="other arguments"):
+            gs.search_counts(ix, *args, **opts)
+    gs.search(ix, (ti, tw), k, path="fused", hybrid=True)
+    cand, resc = gs.search_counts(ix, B, T, k, hybrid=True)
+    assert (cand >= resc).all() and (cand <= 4000).all() and (cand >= k).all()
+    with pytest.raises(ValueError, match="other arguments"):
+        gs.search_counts(ix, B, T, k)
