@@ -35,6 +35,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <numeric>
 #include <type_traits>
 
 #include "gs_topk.h"
@@ -2867,10 +2868,13 @@ int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_
     a.seed = p.seed;
     a.seed_ld = p.seed_docs;
     const int32_t all = (int32_t)((ix->n_docs + kBlkDocs - 1) / kBlkDocs);
-    auto run = [&](bool seed, int32_t b0, int32_t b1) -> int {
-        a.block0 = b0;
-        a.n_blocks = b1 - b0;
-        a.sets = std::min(a.n_blocks, p.lists / p.chunks);
+    a.all = all;
+    a.stride = blk_stride(all);
+    auto run = [&](bool seed, int32_t p0, int32_t p1) -> int {
+        a.place0 = p0;
+        a.n_places = p1 - p0;
+        a.sets = std::min(a.n_places, p.lists / p.chunks);
+        a.hop = (int32_t)((int64_t)a.sets * a.stride % all);
         const unsigned grid = (unsigned)((a.sets * p.chunks + 7) / 8 * 8);
         const size_t lds = blk_lds_fixed(p.Q, bk->n_tail) + (size_t)a.collect * 12;
         if (seed) k_blk_score<true><<<grid, kBlkThreads, lds, s>>>(a);
@@ -2884,20 +2888,21 @@ int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_
     if ((rc = phase(3))) return rc;
     if (o && o->ev_score_begin) GS_CHECK_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(o->ev_score_begin), s));
     // Every doc again, in launches of kBlkGrowth times the docs scored so far, with the
-    // thresholds raised to the k-th of the candidates in between: a launch emits at most
-    // about kBlkGrowth k scores per query.
+    // thresholds raised to the k-th of the candidates in between.  The docs so far lie
+    // all over the collection (blk_stride), so a launch emits about kBlkGrowth k scores
+    // per query and those within the margin below.
     int64_t known = p.seed_docs / kBlkDocs;
-    for (int32_t b0 = 0; b0 < all;) {
-        const int32_t b1 = (int32_t)std::min<int64_t>(all, std::max<int64_t>(b0 + 1, known * kBlkGrowth));
-        if ((rc = run(false, b0, b1))) return rc;
+    for (int32_t p0 = 0; p0 < all;) {
+        const int32_t p1 = (int32_t)std::min<int64_t>(all, std::max<int64_t>(p0 + 1, known * kBlkGrowth));
+        if ((rc = run(false, p0, p1))) return rc;
         k_blk_deal<<<(unsigned)(a.sets * p.chunks), 512, 0, s>>>(p.out_q, p.out_doc, p.out_key, p.out_n, kBlkList,
                                                                  p.chunks, p.Q, p.cap, p.cnt, p.cand_doc, p.cand_key);
         GS_CHECK_LAUNCH();
-        if (b1 < all) {
+        if (p1 < all) {
             k_blk_tau<<<B, 256, 0, s>>>(p.cand_key, p.cap, p.cap, p.cnt, k, p.tau);
             GS_CHECK_LAUNCH();
         }
-        known = b0 = b1;
+        known = p0 = p1;
     }
     if (o && o->ev_score_end) GS_CHECK_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(o->ev_score_end), s));
     if ((rc = phase(4))) return rc;

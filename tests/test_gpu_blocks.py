@@ -228,3 +228,27 @@ def test_block_counts_and_plan(device):
     assert (cand >= resc).all() and (cand <= 4000).all() and (cand >= k).all()
     with pytest.raises(ValueError, match="other arguments"):
         gs.search_counts(ix, B, T, k)
+
+
+@pytest.mark.parametrize("k", [10, 100, 1000])
+def test_block_ordered_collection(device, k):
+    """Documents in the order of their scores, the best last, as a collection in date,
+    length or topical order has them for some queries: the launches' thresholds come
+    from blocks spread over the whole collection, so a query's candidates stay near
+    k per launch (in id order nearly every doc was one)."""
+    rng = np.random.default_rng(k)
+    n, V, B = 60_000, 400, 512
+    rows = np.arange(n, dtype=np.int64)
+    idx = np.stack([np.zeros(n), rng.integers(1, V, size=n)], axis=1).astype(np.int32)
+    w = np.stack([0.5 + rows / n, rng.uniform(0.01, 0.02, size=n)], axis=1).astype(np.float32)
+    csr = gs.CSR(2 * np.arange(n + 1, dtype=np.int64), idx.ravel(), w.ravel(), (n, V))
+    ix = gs.build_from_csr(csr, device)
+    ti = np.stack([np.zeros(B), 1 + np.arange(B) % (V - 1)], axis=1).astype(np.int32)
+    tw = np.stack([rng.uniform(0.5, 2.0, size=B), np.ones(B)], axis=1).astype(np.float32)
+    check(ix, ref_of(csr), ti, tw, k, "ordered")
+    st = {}
+    gs.search(ix, (ti, tw), k, path="fused", timing=st)
+    cand, _ = gs.search_counts(ix, B, 2, k)
+    # about k in each of the at most 5 launches, the docs within the margin (W_0 / 255
+    # of the scores: 0.8% of the docs) and a block's granularity of the samples
+    assert st["dense_rows"] == 0 and cand.max() <= 5 * (2 * k + n * 0.008 + 256)
