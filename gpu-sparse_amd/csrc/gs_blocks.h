@@ -37,6 +37,7 @@ constexpr int kBlkThreads = 512;   // 8 waves, two workgroups per CU
 constexpr int kBlkMinCand = 256;   // emitted scores a workgroup collects in LDS, at least
 constexpr size_t kBlkLds = 80 * 1024 - 64;  // LDS of one of two workgroups on a CU, less the static part
 constexpr int kBlkGroups = 5;      // 64-word groups of a wave whose lookups are in flight together
+constexpr int kBlkClosed = 0x7FFFFFFF;  // threshold of a query that emits nothing: above every score
 constexpr float kBlkTiny = 1e-30f; // lists with a smaller max |w| are scored as zeros
 static_assert(kBlkDocs == 64 && kBlkHeavy % 64 == 0 && kBlkHeavy <= 256, "the kernels' tiles");
 
@@ -464,7 +465,7 @@ __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
     constexpr int KB = kBlkHeavy / 64;
     constexpr int RT = kBlkDocs / 16;
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    __shared__ uint32_t s_nc, s_listed;  // scores collected, and in the workgroup's list
+    __shared__ uint32_t s_nc, s_listed, s_open;  // scores collected, and in the workgroup's list; queries that emit
     unsigned char *tile = lds_raw;
     uint32_t *s_live = reinterpret_cast<uint32_t *>(lds_raw + (size_t)a.Q * (kBlkDocs * 2));
     int32_t *s_thr = reinterpret_cast<int32_t *>(s_live + 2 * blk_live_words(a.n_tail));
@@ -486,20 +487,28 @@ __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
 
     for (int i = tid; i < a.Q * (kBlkDocs * 2 / 16); i += kBlkThreads)
         reinterpret_cast<uint4 *>(tile)[i] = make_uint4(0, 0, 0, 0);
+    if (tid == 0) s_nc = s_listed = s_open = 0;
+    __syncthreads();
     for (int i = tid; i < a.Q; i += kBlkThreads) {
         const int kq = a.kq[q0 + i];
         s_kq[i] = kq;
         s_mul[i] = 1 << a.shift[q0 + i];
-        // the threshold on the products' own scale (kq below the score); slots past B never emit
-        int64_t th = 0x7FFFFFFF;
-        if (!SEED && q0 + i < a.B) th = (int64_t)emit_threshold(a.tau[q0 + i], a.mfix[q0 + i]) - kq;
-        s_thr[i] = (int)(th > 0x7FFFFFFF ? 0x7FFFFFFF : th);
+        // the threshold on the products' own scale (kq below the score); slots past B never
+        // emit, nor do queries past their candidate slots, whose rows are done elsewhere
+        int64_t th = kBlkClosed;
+        if (!SEED && q0 + i < a.B && a.cnt[q0 + i] <= (uint32_t)a.cap)
+            th = (int64_t)emit_threshold(a.tau[q0 + i], a.mfix[q0 + i]) - kq;
+        s_thr[i] = (int)(th > kBlkClosed ? kBlkClosed : th);
+        if (s_thr[i] != kBlkClosed) s_open = 1;
     }
     const int n_live = 2 * blk_live_words(a.n_tail);
     const uint32_t *live = reinterpret_cast<const uint32_t *>(a.live) + (int64_t)chunk * n_live;
     for (int i = tid; i < n_live; i += kBlkThreads) s_live[i] = live[i];
-    if (tid == 0) s_nc = s_listed = 0;
     __syncthreads();
+    if (!SEED && !s_open) {
+        if (tid == 0) a.out_n[lin] = 0;
+        return;
+    }
     const auto r_tab = gs_rsrc(tab, (uint32_t)a.n_tail * 8u);
     const auto r_ent = gs_rsrc(ent, (uint32_t)(a.ent_ld * 4));
 
@@ -516,6 +525,8 @@ __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
         if (slot < (uint32_t)a.cap) {
             a.cand_doc[(int64_t)q * a.cap + slot] = doc;
             a.cand_key[(int64_t)q * a.cap + slot] = key;
+        } else {  // the query is past its slots: no more of it from this workgroup
+            __hip_atomic_store(s_thr + (q - q0), kBlkClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
     };
     // the collected scores to the list; the whole workgroup, after a barrier
@@ -742,7 +753,8 @@ __global__ void __launch_bounds__(256)
     for (int i = tid; i < GS_HIST_BINS; i += 256) s_hist[i] = 0;
     __syncthreads();
     const uint32_t *row = score + (int64_t)q * ld;
-    const int m = cnt ? (int)min(cnt[q], (uint32_t)n) : n;
+    if (cnt && cnt[q] > (uint32_t)n) return;  // past its slots: k_blk_score emits nothing of it
+    const int m = cnt ? (int)cnt[q] : n;
     for (int i0 = tid; i0 < m; i0 += 256 * 8) {
         uint32_t v[8];
 #pragma unroll

@@ -252,3 +252,31 @@ def test_block_ordered_collection(device, k):
     # about k in each of the at most 5 launches, the docs within the margin (W_0 / 255
     # of the scores: 0.8% of the docs) and a block's granularity of the samples
     assert st["dense_rows"] == 0 and cand.max() <= 5 * (2 * k + n * 0.008 + 256)
+
+
+def one_term_csr(n, weight, vocab=50):
+    """n docs that all hold term 0 with the given weights and one other term, weakly."""
+    idx = np.stack([np.zeros(n), 1 + np.arange(n) % (vocab - 1)], axis=1).astype(np.int32)
+    w = np.stack([np.broadcast_to(weight, n), np.full(n, 0.001)], axis=1).astype(np.float32)
+    return gs.CSR(2 * np.arange(n + 1, dtype=np.int64), idx.ravel(), w.ravel(), (n, vocab))
+
+
+@pytest.mark.parametrize("n,k", [(16_000, 100), (16_000, 1000), (70_000, 100)])
+def test_block_list_overflow(device, n, k):
+    """One block emits 64 docs x 512 queries, twice what a workgroup's list holds: the
+    rest goes straight to the queries' candidates.  16000 tied docs fit a query's
+    slots and its rescoring; of 70000 a query takes what fits its slots, emits no
+    more, and its row is done elsewhere."""
+    B = 512
+    csr = one_term_csr(n, 1.0)
+    ix = gs.build_from_csr(csr, device)
+    ti = np.zeros((B, 1), np.int32)
+    tw = np.linspace(0.5, 2.0, B, dtype=np.float32)[:, None]
+    check(ix, ref_of(csr), ti, tw, k, f"list overflow n={n}")
+    st = {}
+    gs.search(ix, (ti, tw), k, path="fused", timing=st)
+    if n == 16_000:
+        cand, resc = gs.search_counts(ix, B, 1, k)
+        assert st["dense_rows"] == 0 and (cand == n).all() and (resc == n).all()
+    else:
+        assert st["dense_rows"] == B
