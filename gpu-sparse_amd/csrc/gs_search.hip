@@ -2734,6 +2734,17 @@ BlkPlan plan_blocks(const gs_index *ix, const gs_block_copy *bk, int32_t B, int3
     sd = (std::min<int64_t>(sd, ix->n_docs) + kBlkDocs - 1) / kBlkDocs * kBlkDocs;
     p.seed_docs = (int32_t)sd;
     p.cap = cand_slots(ix, B, k, o);
+    if (!(o && o->cand_cap > 0)) {
+        // The scoring launches emit about 2 k scores, then k each, and those within the
+        // margin: 2.5 k for the start and for each doubling of the docs hold them.  512
+        // queries on 8.8M docs at k = 8192 emit 89K each, at most 114K: with the default's
+        // 66K slots all rows went to the dense path, 159 ms instead of 10.0.  At most 4 GiB
+        // of slots where the default has fewer.
+        int64_t doublings = 0;
+        while ((sd << doublings) < ix->n_docs) ++doublings;
+        const int64_t want = std::min<int64_t>((ix->n_docs + 255) / 256 * 256, 5ll * k * (2 + doublings) / 2);
+        p.cap = (int32_t)std::max<int64_t>(p.cap, std::min<int64_t>(want, std::min<int64_t>(kMaxCandCap, (1ll << 29) / B)));
+    }
     p.rcap = kRescoreCap;
     p.ent_ld = (int64_t)p.Q * T + 8;  // + 8: entries are read four and eight at a time
     p.mfix = ar.take<uint32_t>(B);

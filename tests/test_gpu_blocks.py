@@ -280,3 +280,25 @@ def test_block_list_overflow(device, n, k):
         assert st["dense_rows"] == 0 and (cand == n).all() and (resc == n).all()
     else:
         assert st["dense_rows"] == B
+
+
+def test_block_large_k_slots(device):
+    """The most results of the fused path on a collection of several launches: the
+    queries' slots hold what all of them emit (65536 did not)."""
+    rng = np.random.default_rng(5)
+    n, B, k = 6_000_000, 512, 8192
+    csr = one_term_csr(n, rng.lognormal(-0.5, 0.8, size=n))
+    ix = gs.build_from_csr(csr, device)
+    ti = np.zeros((B, 1), np.int32)
+    tw = np.linspace(0.5, 2.0, B, dtype=np.float32)[:, None]
+    st = {}
+    s, i = gs.search(ix, (ti, tw), k, path="fused", timing=st)
+    assert gs.search_plan(ix, B, 1, k)["blocks"] and st["dense_rows"] == 0
+    cand, _ = gs.search_counts(ix, B, 1, k)
+    assert (cand >= k).all() and cand.max() > 65536
+    w = csr.data[0::2].astype(np.float64)
+    for q in (0, 255, 511):
+        exact = w * float(tw[q, 0])
+        best = np.lexsort((np.arange(n), -exact))[:k]
+        assert np.array_equal(i[q].cpu().numpy(), best)
+        assert np.array_equal(s[q].cpu().numpy(), exact[best].astype(np.float32))
