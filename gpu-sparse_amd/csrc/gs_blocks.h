@@ -38,6 +38,7 @@ constexpr int kBlkMinCand = 256;   // emitted scores a workgroup collects in LDS
 constexpr size_t kBlkLds = 80 * 1024 - 64;  // LDS of one of two workgroups on a CU, less the static part
 constexpr int kBlkGroups = 5;      // 64-word groups of a wave whose lookups are in flight together
 constexpr int kBlkClosed = 0x7FFFFFFF;  // threshold of a query that emits nothing: above every score
+constexpr uint32_t kBlkPast = 0xFFFFFFFFu;  // candidate count of a query that is given up: past any slots
 constexpr float kBlkTiny = 1e-30f; // lists with a smaller max |w| are scored as zeros
 static_assert(kBlkDocs == 64 && kBlkHeavy % 64 == 0 && kBlkHeavy <= 256, "the kernels' tiles");
 
@@ -192,8 +193,9 @@ struct BlkQueries {
 
 // One wave per query slot: C, r and Ct (top of the file), the heavy limbs, the
 // margin, the counts of the tail terms' entries.  Slots past B get zero limbs, and
-// so do queries without a feasible C (non-finite weights, no term, too many
-// terms), whose margin 2^31 - 1 sends their row to the dense path.
+// so do queries without a feasible C: non-finite weights and no term, whose margin
+// 2^31 - 1 and lack of candidates send their row to the dense path, and too many
+// terms or too wide a margin, whose row is flagged as past its candidate slots.
 __global__ void __launch_bounds__(256) k_blk_prep(const BlkQueries a) {
     __shared__ double s_q[4][kBlkHeavy];
     const int wv = threadIdx.x >> 6;
@@ -311,7 +313,7 @@ __global__ void __launch_bounds__(256) k_blk_prep(const BlkQueries a) {
         a.ct[q] = ok ? Ct : 0.0;
         a.mfix[q] = ok ? (uint32_t)mf : 0x7FFFFFFFu;
         a.tau[q] = 0;
-        a.cnt[q] = 0;
+        a.cnt[q] = !ok && M > 0.0 && M < inf ? kBlkPast : 0;
     }
     if (!ok) return;
     uint2 *tab = a.tab + (int64_t)(q / a.Q) * (a.n_tail + 1);

@@ -1895,13 +1895,15 @@ __global__ void __launch_bounds__(256)
 // uint8 rows: the exact top-k of the candidates is the answer.  Float rows: the
 // fixed-point k-th score tau' gives the rescoring set {fixed >= tau' - mfix};
 // nothing is sorted, and the first `held` keys stay in dynamic LDS over the passes.
+// `wide`: the status of a row that overflows its slots or is not clear of zero, as a
+// narrower margin could settle it (rows with fewer than k candidates need the dense path).
 template <int WT>
 __global__ void __launch_bounds__(kSelThreads, WT == GS_W_U8 ? 4 : 8)
     k_select_cands(const uint32_t *__restrict__ cand_doc, const uint32_t *__restrict__ cand_key,
                    const uint32_t *__restrict__ cnt, int32_t cap, int32_t k, int32_t held, const uint32_t *__restrict__ mfix,
                    uint32_t *__restrict__ resc_doc, uint32_t *__restrict__ resc_cnt, int32_t resc_cap,
                    const int32_t *__restrict__ perm, void *__restrict__ out_scores, int64_t *__restrict__ out_ids,
-                   int32_t *__restrict__ status) {
+                   int32_t *__restrict__ status, int32_t wide) {
     constexpr bool FP = WT != GS_W_U8;
     __shared__ SelStatic sst;
     SelShared sh = sel_view(sst, k);
@@ -1911,7 +1913,7 @@ __global__ void __launch_bounds__(kSelThreads, WT == GS_W_U8 ? 4 : 8)
     const uint32_t n = cnt[q];
     if (n > (uint32_t)cap || n < (uint32_t)k) {
         if (threadIdx.x == 0) {
-            status[row] = GS_ROW_DENSE;
+            status[row] = n > (uint32_t)cap ? wide : GS_ROW_DENSE;
             if (FP) resc_cnt[q] = 0;
         }
         return;
@@ -1932,7 +1934,7 @@ __global__ void __launch_bounds__(kSelThreads, WT == GS_W_U8 ? 4 : 8)
         const uint32_t mf = mfix[q];
         if (kth <= mf) {  // k-th score not clear of zero by the margin
             if (threadIdx.x == 0) {
-                status[row] = GS_ROW_DENSE;
+                status[row] = wide;
                 resc_cnt[q] = 0;
             }
             return;
@@ -1949,7 +1951,7 @@ __global__ void __launch_bounds__(kSelThreads, WT == GS_W_U8 ? 4 : 8)
         if (threadIdx.x == 0) {
             const uint32_t m = s_m;
             if (m > (uint32_t)resc_cap) {
-                status[row] = GS_ROW_DENSE;
+                status[row] = wide;
                 resc_cnt[q] = 0;
             } else {
                 status[row] = GS_ROW_DONE;
@@ -2511,7 +2513,7 @@ DenseRow dense_row(const gs_index *ix, size_t acc_bytes) {
 template <int WT, class Plan, class Phase>
 int select_and_rescore(const gs_index *ix, const int32_t *qt, const void *qw, int32_t B, int32_t T, int32_t k,
                        const Plan &p, const int32_t *perm, void *out_scores, int64_t *out_ids, int32_t *status,
-                       Phase &&phase, hipStream_t s) {
+                       int32_t wide, Phase &&phase, hipStream_t s) {
     constexpr bool FP = WT != GS_W_U8;
     int rc = GS_OK;
     const size_t sel_lds = sel_lds_bytes(k);
@@ -2523,7 +2525,7 @@ int select_and_rescore(const gs_index *ix, const int32_t *qt, const void *qw, in
     GS_CHECK_HIP(sel_attr((const void *)k_select_cands<WT>, cand_lds));
     k_select_cands<WT><<<B, kSelThreads, cand_lds, s>>>(p.cand_doc, p.cand_key, p.cnt, p.cap, k, held, p.mfix,
                                                         p.resc_doc, p.resc_cnt, p.rcap, perm, out_scores, out_ids,
-                                                        status);
+                                                        status, wide);
     GS_CHECK_LAUNCH();
     if ((rc = phase(5))) return rc;
     if (FP) {
@@ -2692,7 +2694,9 @@ int search_impl(const gs_index *ix, const int32_t *qt, const void *qw, int32_t B
     }
     if ((rc = phase(4))) return rc;
 
-    if ((rc = select_and_rescore<WT>(ix, qt, qw, B, T, k, p, perm, out_scores, out_ids, status, phase, s))) return rc;
+    if ((rc = select_and_rescore<WT>(ix, qt, qw, B, T, k, p, perm, out_scores, out_ids, status, GS_ROW_DENSE,
+                                     phase, s)))
+        return rc;
     return phase(7);
 }
 
@@ -2917,7 +2921,9 @@ int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_
     }
     if (o && o->ev_score_end) GS_CHECK_HIP(hipEventRecord(reinterpret_cast<hipEvent_t>(o->ev_score_end), s));
     if ((rc = phase(4))) return rc;
-    if ((rc = select_and_rescore<WT>(ix, qt, qw, B, T, k, p, nullptr, out_scores, out_ids, status, phase, s))) return rc;
+    if ((rc = select_and_rescore<WT>(ix, qt, qw, B, T, k, p, nullptr, out_scores, out_ids, status, GS_ROW_RETRY,
+                                     phase, s)))
+        return rc;
     return phase(7);
 }
 

@@ -19,7 +19,7 @@ SYNTH_PATH = os.path.join(_HERE, "libgs_synth.so")
 
 GS_OK, GS_EINVAL, GS_EHIP, GS_ENOSPC = 0, 1, 2, 3
 GS_W_F32, GS_W_F16, GS_W_U8 = 0, 1, 2
-GS_ROW_DONE, GS_ROW_DENSE = 0, 1
+GS_ROW_DONE, GS_ROW_DENSE, GS_ROW_RETRY = 0, 1, 2
 GS_SEARCH_PHASES = 8
 NOALLOC_SCRATCH_BYTES = 256 << 20   # GS_NOALLOC_SCRATCH_BYTES
 PHASE_NAMES = ("query_prep", "heavy_terms", "threshold_seed", "scoring", "candidate_select", "fp64_rescore",

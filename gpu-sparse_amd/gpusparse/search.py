@@ -266,8 +266,9 @@ class PendingSearch:
     """A search whose kernels are queued on a stream (`search_async`).
 
     `result()` waits for the fused pipeline's per-row status (one event, no
-    device-wide synchronisation), finishes the rows it flagged with the dense
-    path on the same stream and returns ``(scores [B, k], ids [B, k] int64)``.
+    device-wide synchronisation), finishes the rows it flagged on the same stream
+    (with the dense path; those of a block search first as a batch of their own,
+    which it waits for) and returns ``(scores [B, k], ids [B, k] int64)``.
     The returned tensors are ordered on the search's stream: the stream current
     at the `result()` call is made to wait for it."""
 
@@ -282,16 +283,16 @@ class PendingSearch:
         self._post = post  # applied to the results once, on the stream current at result()
 
     def done(self) -> bool:
-        """True when result() would not wait for the GPU."""
+        """True when result() would not wait for this search (it does for the rows
+        that a block search leaves to a second one)."""
         return self._finish is None or self._event.query()
 
     def result(self):
         if self._finish is not None:
             self._event.synchronize()
-            bad = np.nonzero(self._status_h.numpy() != _lib.GS_ROW_DONE)[0]
+            status, self._status_h = self._status_h.numpy(), None
             finish, self._finish = self._finish, None
-            self._status_h = None
-            finish(bad)
+            finish(status)
         if self._stream is not None:
             cur = torch.cuda.current_stream(self._stream.device)
             if cur != self._stream:
@@ -323,7 +324,8 @@ def search(index, query_batch, k: int = 10, *, tile_log2: int | None = None, pat
     the GS_SEARCH_PHASES events of each call ("phases": start, query prep,
     heavy-term sums, threshold seed, scoring, candidate selection, fp64
     rescoring, final sort) and
-    the number of rows finished by the dense path ("dense_rows").  Events come
+    the number of rows finished by the dense path ("dense_rows") and of those a
+    block search left to a second search ("retried_rows").  Events come
     from timing["event_pool"] while it lasts (see `timing_dict`).
     batch_order: score queries in groups of consecutive queries instead of groups of
     queries sharing frequent terms (same results; for comparisons)."""
@@ -448,11 +450,29 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
     done = torch.cuda.Event()
     done.record(stream)
 
-    def finish(bad):
+    def finish(status):
         if bad_h is not None and bool(bad_h):
             raise ValueError(_U8_WEIGHTS_MSG)
+        bad = np.nonzero((status != _lib.GS_ROW_DONE) & (status != _lib.GS_ROW_RETRY))[0]
+        retry = np.nonzero(status == _lib.GS_ROW_RETRY)[0]
+        dense = int(bad.size)
+        if retry.size:
+            # Rows the block search's margin did not settle: a batch of their own, dense
+            # or hybrid by the same rule, as its cost per row is a small part of the dense
+            # path's where many are flagged (64 of 512 queries of 300 terms on 1M docs
+            # added 14 ms as dense rows, 1 as a hybrid batch)
+            with torch.cuda.stream(stream):
+                rows = torch.from_numpy(retry).to(dev)
+                again = None if timing is None else {}
+                s2, i2 = search_async(index, (qt[rows], qw[rows]), kk, tile_log2=tile_log2, hybrid=hyb,
+                                      dense_budget=dense_budget, timing=again).result()
+                out_s.index_copy_(0, rows, s2)
+                out_i.index_copy_(0, rows, i2)
+            if timing is not None:
+                dense += again.get("dense_rows", int(retry.size))
         if timing is not None:
-            timing["dense_rows"] = timing.get("dense_rows", 0) + int(bad.size)
+            timing["dense_rows"] = timing.get("dense_rows", 0) + dense
+            timing["retried_rows"] = timing.get("retried_rows", 0) + int(retry.size)
         if bad.size:
             with torch.cuda.stream(stream):
                 rows = torch.from_numpy(bad.astype(np.int32)).to(dev)

@@ -40,6 +40,8 @@ extern "C" {
 /* Per-query status written by gs_search. */
 #define GS_ROW_DONE 0
 #define GS_ROW_DENSE 1  /* row must be finished by gs_search_dense (rare: overflow or < k positive scores) */
+#define GS_ROW_RETRY 2  /* of gs_search_blocks alone: the block scorer's margin does not settle the row; gs_search
+                         * may (its margin is narrower), gs_search_dense does */
 
 /*
  * Device-resident term-major inverted index: the layout of the reference's
@@ -308,8 +310,8 @@ int gs_blocks_fill(const int64_t *fwd_ptr_d, const int32_t *fwd_terms_d, const v
                    int64_t n_docs, int32_t vocab, const int32_t *rank_d, const float *max_abs_d, int32_t levels,
                    int8_t *head_d, uint32_t *tail_d, int32_t *count_d, int32_t *negative_d, void *workspace_d,
                    void *stream);
-/* As gs_search (same results, status, phases and score events; of the options only
- * cand_cap and the events apply).  Of the index it reads n_docs, vocab, wtype,
+/* As gs_search (same results, phases and score events, the status GS_ROW_RETRY beside
+ * gs_search's two; of the options only cand_cap and the events apply).  Of the index it reads n_docs, vocab, wtype,
  * max_abs_d, dup_d and the doc-major copy. */
 int gs_search_blocks_workspace(const gs_index *index, const gs_block_copy *blocks, int32_t B, int32_t T, int32_t k,
                                const gs_search_opts *opts, size_t *bytes);

@@ -302,3 +302,33 @@ def test_block_large_k_slots(device):
         best = np.lexsort((np.arange(n), -exact))[:k]
         assert np.array_equal(i[q].cpu().numpy(), best)
         assert np.array_equal(s[q].cpu().numpy(), exact[best].astype(np.float32))
+
+
+def outlier_csr(rng, n, vocab, per_row, times):
+    """n docs of per_row distinct terms of `vocab`, and in each list one weight `times`
+    the largest other."""
+    idx = np.sort(np.argpartition(rng.random((n, vocab), dtype=np.float32), per_row, axis=1)[:, :per_row], axis=1)
+    w = rng.uniform(0.5, 1.0, size=(n, per_row)).astype(np.float32)
+    flat, first = idx.ravel(), np.unique(idx.ravel(), return_index=True)[1]
+    assert first.size == vocab and flat.size == n * per_row
+    w.ravel()[first] = times
+    return gs.CSR(per_row * np.arange(n + 1, dtype=np.int64), flat.astype(np.int32), w.ravel(), (n, vocab))
+
+
+@pytest.mark.parametrize("B", [20, 300])
+def test_block_margin_too_wide(device, B):
+    """Lists with one weight far above the rest: the block copy's levels, relative to a
+    list's largest weight, leave more docs within the margin than are rescored.  Such
+    rows are searched once more as a batch of their own (300 queries: by the hybrid
+    scorer, whose margin settles them; 20: as dense rows), not one by one densely."""
+    rng = np.random.default_rng(B)
+    n, V, k = 60_000, 160, 500
+    csr = outlier_csr(rng, n, V, 24, 200.0)
+    ix = gs.build_from_csr(csr, device)
+    ti, tw = random_queries(rng, B, V, max_len=10)
+    ti[:, 0], tw[:, 0] = rng.integers(0, V, size=B), 1.0
+    st = {}
+    check(ix, ref_of(csr), ti, tw, k, "outliers")
+    s, i = gs.search(ix, (ti, tw), k, path="fused", timing=st)
+    assert st["retried_rows"] > B // 2
+    assert st["dense_rows"] < st["retried_rows"] // 4 if B == 300 else st["dense_rows"] >= st["retried_rows"]
