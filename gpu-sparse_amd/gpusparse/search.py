@@ -370,18 +370,24 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
     # selection takes any k (rounds of MAX_K) and whose scorer any width
     if path == "dense" or kk > MAX_K or T > MAX_T or (path == "auto" and dense_preferred(index, B, kk, tile_log2, hyb,
                                                                                         dense_budget)):
-        late = hyb and index.wtype == _lib.GS_W_U8  # the weights' check is read with the results
-        if bad_w is not None and not late and bool(bad_w):
-            raise ValueError(_U8_WEIGHTS_MSG)
+        done = bad_h = finish = None
+        if bad_w is not None:
+            if not (hyb and index.wtype == _lib.GS_W_U8):
+                if bool(bad_w):
+                    raise ValueError(_U8_WEIGHTS_MSG)
+            else:  # the weights' check is read with the results, which wait for it alone
+                bad_h = torch.empty((), dtype=torch.bool, pin_memory=True)
+                bad_h.copy_(bad_w, non_blocking=True)
+                done = torch.cuda.Event()
+                done.record(stream)
+
+                def finish(bad):
+                    if bool(bad):
+                        raise ValueError(_U8_WEIGHTS_MSG)
+
         gidx = gs_index_struct(index, tile_log2, scorer=False)
         _dense_rows(index, gidx, qt, qw, kk, None, out_s, out_i, max(dense_budget, 1))
-
-        def checked(out):
-            if bool(bad_w):
-                raise ValueError(_U8_WEIGHTS_MSG)
-            return out
-
-        return PendingSearch((out_s, out_i), stream, post=checked if late and bad_w is not None else None)
+        return PendingSearch((out_s, out_i), stream, done, bad_h, finish)
     if hyb and index.wtype == _lib.GS_W_U8:
         # the float16 copy's hybrid search; its fp32 scores are the exact sums.
         # The weights' check (device weights) is copied out ahead of the search,

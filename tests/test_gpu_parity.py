@@ -885,6 +885,33 @@ def test_reference_builders_store_float32(device, dtype):
             gs.search(native, (torch.from_numpy(ti).cuda(), torch.from_numpy(tw - 300).cuda()), 20, path="dense")
 
 
+def test_done_of_a_dense_search(device):
+    """done() of a dense uint8 search with weights on the GPU: false while result() would
+    wait for their check."""
+    rng = np.random.default_rng(43)
+    csr = random_csr(rng, 2000, 300, max_len=12, dtype=np.uint8)
+    ix = gs.build_index(csr, device, weight_dtype=torch.uint8)
+    ti, tw = random_queries(rng, 4, 300, max_len=8, dtype=np.uint8)
+    good = torch.from_numpy(ti).cuda(), torch.from_numpy(tw.astype(np.float32)).cuda()
+    want = gs.search(ix, good, 10, path="dense")
+    bad = good[0], good[1] + 0.5
+    x = torch.ones(8192, 8192, device=device)
+    torch.cuda.synchronize()
+    for q in (good, bad):
+        for _ in range(20):  # some 0.2 s of work ahead of the search
+            y = x @ x
+        p = gs.search_async(ix, q, 10, path="dense")
+        assert not p.done()
+        if q is bad:
+            with pytest.raises(ValueError, match="integers"):
+                p.result()
+        else:
+            s, i = p.result()
+            assert torch.equal(s, want[0]) and torch.equal(i, want[1])
+        assert p.done()
+    del y
+
+
 def test_retrieve_and_run_engine(device, tmp_path):
     rng = np.random.default_rng(41)
     csr = random_csr(rng, 3000, 400, max_len=20, sort_rows=True)
