@@ -2710,7 +2710,6 @@ constexpr int kBlkList = 16384;          // emitted scores a workgroup's list ho
 struct BlkPlan {
     int32_t chunks, Q, slots, seed_docs, cap, rcap;
     int64_t ent_ld;
-    float *scale;
     uint32_t *mfix, *tau, *cnt, *cand_doc, *cand_key, *resc_doc, *resc_cnt;
     uint64_t *resc_key;
     int8_t *alimb;
@@ -2755,7 +2754,7 @@ BlkPlan plan_blocks(const gs_index *ix, const gs_block_copy *bk, int32_t B, int3
     p.tau = ar.take<uint32_t>(B);
     p.cnt = ar.take<uint32_t>(B);
     p.resc_cnt = ar.take<uint32_t>(B);
-    p.cleared = (int64_t)p.chunks * (bk->n_tail + 1) * 2 + p.chunks;
+    p.cleared = (int64_t)p.chunks * bk->n_tail * 2 + p.chunks;
     uint32_t *cleared = ar.take<uint32_t>((size_t)p.cleared);
     p.tab = reinterpret_cast<uint2 *>(cleared);
     p.total = cleared ? cleared + (size_t)(p.cleared - p.chunks) : nullptr;

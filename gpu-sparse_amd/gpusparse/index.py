@@ -18,7 +18,9 @@ from dataclasses import dataclass, field
 from typing import Any, NamedTuple
 
 import ctypes as C
+import functools
 import math
+import threading
 
 import numpy as np
 import torch
@@ -288,6 +290,22 @@ def build_gpu_inverted_index_from_sparse(sparse_matrix, device=torch.device("cud
 # ------------------------------------------------------------------ checks and bounds
 
 
+# Held while an index's derived state is built: arrays are published in aux() before
+# their kernels have run, and a thread on another stream must not read them until the
+# builder has waited for its own.  Once the state is there it is held for a few
+# dictionary look-ups.
+_state_lock = threading.RLock()
+
+
+def state_locked(f):
+    """Calls f with the lock of the indexes' derived state held (reentrant)."""
+    @functools.wraps(f)
+    def locked(*args, **kwargs):
+        with _state_lock:
+            return f(*args, **kwargs)
+    return locked
+
+
 def check_lists(index) -> tuple[int, int]:
     """(non-ascending lists, non-empty lists); caches the per-list duplicate counts."""
     dev = _device_of(index)
@@ -367,6 +385,7 @@ def heavy_terms(index) -> torch.Tensor:
     return out
 
 
+@state_locked
 def hybrid_eligible(index) -> bool:
     """Whether the hybrid search can serve the index: float weights with a packed
     copy (finite weights), and heavy lists that hold each doc at most once.
@@ -405,6 +424,7 @@ def build_head(index):
     return head, rank
 
 
+@state_locked
 def ensure_search_state(index, tile_log2: int | None = None, forward: bool = True, hybrid: bool = False,
                         scorer: bool = True) -> dict:
     """Derived arrays gs_search needs: max |w|, duplicate counts, the most frequent
@@ -480,6 +500,7 @@ class Blocks(NamedTuple):
         return _lib.GsBlockCopy(*(t.data_ptr() for t in self[:5]), self.n_tail, self.levels)
 
 
+@state_locked
 def blocks_eligible(index) -> bool:
     """Whether the block search can serve the index: float weights, all finite, the
     128 longest lists holding each doc once, at most 65535 further non-empty lists."""
@@ -500,6 +521,7 @@ def blocks_eligible(index) -> bool:
     return a["blocks_ok"]
 
 
+@state_locked
 def ensure_blocks(index) -> Blocks | None:
     """The block copy of an eligible index and the doc-major copy it is made from,
     built once; None when the GPU has no room for them (the search then takes the
@@ -539,6 +561,7 @@ def ensure_blocks(index) -> Blocks | None:
         torch.cuda.current_stream(dev).synchronize()
         a["blocks"] = Blocks(head, tail, count, rank_d, heavy_d, max(order.size - _lib.BLOCK_HEAVY, 1), levels)
     except torch.cuda.OutOfMemoryError:
+        torch.cuda.current_stream(dev).synchronize()  # the doc-major copy may stand
         a["blocks"] = None
     return a["blocks"]
 

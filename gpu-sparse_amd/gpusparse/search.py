@@ -22,7 +22,8 @@ import torch
 
 from . import _lib
 from .index import (DEFAULT_TILE_LOG2_HYBRID, blocks_eligible, default_tile_log2, ensure_blocks, gs_blocks_index,
-                    gs_index_struct, hybrid_eligible, _device_of)
+                    gs_index_struct, hybrid_eligible, _device_of,
+                    state_locked)
 
 MAX_K = 8192  # largest k of the fused path and of compacted_topk; search answers larger k densely
 MAX_T = 8192  # widest query batch of the fused path (terms per query); search answers wider ones densely
@@ -94,6 +95,7 @@ HYBRID_DEFAULT = True  # whether searches that name no scorer take the hybrid on
 U8_HYBRID_MAX_T = 258  # widest uint8 batch the float16 copy serves: 258 * 255 * 255 < 2^24
 
 
+@state_locked
 def u8_float_copy(index):
     """For a uint8 index: the same postings with the weights as float16 (exact
     for 0..255), which the hybrid search runs on; built once, kept in aux()
@@ -112,6 +114,7 @@ def u8_float_copy(index):
     return f
 
 
+@state_locked
 def u8_hybrid_ok(index, T: int | None = None) -> bool:
     """Whether a uint8 index can take the hybrid search through its float16 copy
     for batches T terms wide: no list repeats a doc (so a doc's sum holds at

@@ -2,6 +2,7 @@
 terms added in an LDS tile) against the oracle: block, chunk and group edges,
 signs, repeated terms, and its copy's levels and words."""
 import sys
+import threading
 
 import numpy as np
 import pytest
@@ -191,6 +192,7 @@ def test_block_configs(device, cfg, n_docs, B, k):
     ti, tw, _ = O.to_query_tensors(queries.indptr, queries.indices, queries.data)
     if cfg == "C5":
         tw = tw.astype(np.uint8)
+        assert gs.search_plan(ix, B, ti.shape[1], k)["blocks"]
         s, i = gs.search(ix, (ti, tw), k, path="fused")
         es, ei = O.search(ref, ti, tw, k)
         assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(s.cpu().numpy(), es)
@@ -332,3 +334,57 @@ def test_block_margin_too_wide(device, B):
     s, i = gs.search(ix, (ti, tw), k, path="fused", timing=st)
     assert st["retried_rows"] > B // 2
     assert st["dense_rows"] < st["retried_rows"] // 4 if B == 300 else st["dense_rows"] >= st["retried_rows"]
+
+
+def test_block_copy_threads(device, monkeypatch):
+    """Threads that search a new index at once, each on a stream of its own: the block copy
+    is made once, and no thread reads it before it is whole."""
+    rng = np.random.default_rng(31)
+    csr = head_tail_csr(rng, 20_000, 3000, np.float16)
+    ref = ref_of(csr)
+    batches = [random_queries(rng, 30 + 40 * i, 3000, max_len=20) for i in range(4)]
+    module = sys.modules["gpusparse.index"]
+    builds, blocks = [], module.Blocks
+    monkeypatch.setattr(module, "Blocks", lambda *a: builds.append(1) or blocks(*a))
+    for trial in range(3):
+        ix = gs.build_from_csr(csr, device)
+        if trial:
+            ix.aux().pop("fwd")  # the doc-major copy made with the blocks, not the uploaded CSR
+        torch.cuda.synchronize()
+        got, start = [None] * 4, threading.Barrier(4)
+
+        def work(i):
+            with torch.cuda.stream(torch.cuda.Stream(device)):
+                start.wait(60)
+                got[i] = [x.cpu().numpy() for x in gs.search(ix, batches[i], 100, path="fused")]
+
+        builds.clear()
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert len(builds) == 1 and ix.aux()["blocks"] is not None
+        for (ti, tw), out in zip(batches, got):
+            es, _, ei = O.c_search(ref, ti, tw, 100, threads=8)
+            assert np.array_equal(out[1], ei) and np.array_equal(out[0], es)
+
+
+def test_block_streams(device):
+    """Batches of different sizes in flight on two streams, each with a workspace of its own."""
+    rng = np.random.default_rng(32)
+    csr = head_tail_csr(rng, 30_000, 3000, np.float32)
+    ix, ref = gs.build_from_csr(csr, device), ref_of(csr)
+    streams = [torch.cuda.Stream(device) for _ in range(2)]
+    jobs = [(*random_queries(rng, B, 3000, max_len=T), k) for B, T, k in
+            ((512, 30, 100), (17, 8, 1000), (300, 60, 10), (1, 30, 500), (600, 20, 50), (64, 5, 1))]
+    want = [O.c_search(ref, ti, tw, k, threads=8) for ti, tw, k in jobs]
+    assert gs.search_plan(ix, 17, 8, 1000)["blocks"]
+    for r in range(3):
+        pending = []
+        for i, (ti, tw, k) in enumerate(jobs):
+            with torch.cuda.stream(streams[(i + r) % 2]):
+                pending.append(gs.search_async(ix, (ti, tw), k, path="fused"))
+        for p, (es, _, ei) in zip(pending, want):
+            s, i = p.result()
+            assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(s.cpu().numpy(), es)
