@@ -16,6 +16,7 @@ float32; uint8 indexes return the exact uint32 sums as int32.
 from __future__ import annotations
 
 from collections import OrderedDict
+from contextlib import contextmanager
 
 import numpy as np
 import torch
@@ -193,6 +194,22 @@ def _workspace(index, nbytes: int, stream_key: int = 0, plan=None) -> torch.Tens
         pool.popitem(last=False)
     a["workspace"], a["workspace_plan"] = ws, plan
     return ws
+
+
+@contextmanager
+def _workspace_aside(index, stream_key: int):
+    """Lays the index's workspace for a stream aside: a search inside gets one of its own,
+    dropped at the end, and search_counts goes on reading the one laid aside."""
+    a = index.aux()
+    kept = {n: a.get(n) for n in ("workspace", "workspace_plan")}
+    ws = a["workspaces"].pop(stream_key, None)
+    try:
+        yield
+    finally:
+        a["workspaces"].pop(stream_key, None)
+        if ws is not None:
+            a["workspaces"][stream_key] = ws
+        a.update(kept)
 
 
 def _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch_order) -> bool:
@@ -464,21 +481,24 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
             raise ValueError(_U8_WEIGHTS_MSG)
         bad = np.nonzero((status != _lib.GS_ROW_DONE) & (status != _lib.GS_ROW_RETRY))[0]
         retry = np.nonzero(status == _lib.GS_ROW_RETRY)[0]
-        dense = int(bad.size)
+        again = {}
         if retry.size:
             # Rows the block search's margin did not settle: a batch of their own, dense
             # or hybrid by the same rule, as its cost per row is a small part of the dense
             # path's where many are flagged (64 of 512 queries of 300 terms on 1M docs
-            # added 14 ms as dense rows, 1 as a hybrid batch)
-            with torch.cuda.stream(stream):
+            # added 14 ms as dense rows, 1 as a hybrid batch); as dense rows, a few at a
+            # time, where the GPU has no room for that
+            with torch.cuda.stream(stream), _workspace_aside(index, stream.cuda_stream):
                 rows = torch.from_numpy(retry).to(dev)
-                again = None if timing is None else {}
-                s2, i2 = search_async(index, (qt[rows], qw[rows]), kk, tile_log2=tile_log2, hybrid=hyb,
-                                      dense_budget=dense_budget, timing=again).result()
-                out_s.index_copy_(0, rows, s2)
-                out_i.index_copy_(0, rows, i2)
-            if timing is not None:
-                dense += again.get("dense_rows", int(retry.size))
+                try:
+                    s2, i2 = search_async(index, (qt[rows], qw[rows]), kk, tile_log2=tile_log2, hybrid=hyb,
+                                          dense_budget=dense_budget, timing=None if timing is None else again).result()
+                    out_s.index_copy_(0, rows, s2)
+                    out_i.index_copy_(0, rows, i2)
+                except torch.cuda.OutOfMemoryError:
+                    bad = np.sort(np.concatenate([bad, retry]))
+                    again["dense_rows"] = 0
+        dense = int(bad.size) + (again.get("dense_rows", int(retry.size)) if retry.size else 0)
         if timing is not None:
             timing["dense_rows"] = timing.get("dense_rows", 0) + dense
             timing["retried_rows"] = timing.get("retried_rows", 0) + int(retry.size)

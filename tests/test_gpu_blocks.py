@@ -334,6 +334,32 @@ def test_block_margin_too_wide(device, B):
     s, i = gs.search(ix, (ti, tw), k, path="fused", timing=st)
     assert st["retried_rows"] > B // 2
     assert st["dense_rows"] < st["retried_rows"] // 4 if B == 300 else st["dense_rows"] >= st["retried_rows"]
+    # the counts are the block search's own, not those of the rows searched again
+    cand, resc = gs.search_counts(ix, B, ti.shape[1], k)
+    assert (cand >= k).sum() >= st["retried_rows"] and (resc == 0).sum() >= st["retried_rows"]
+
+
+def test_block_retry_without_room(device, monkeypatch):
+    """Rows to search again that the GPU has no workspace for: dense rows."""
+    rng = np.random.default_rng(300)
+    n, V, k, B = 60_000, 160, 500, 300
+    csr = outlier_csr(rng, n, V, 24, 200.0)
+    ix = gs.build_from_csr(csr, device)
+    ti, tw = random_queries(rng, B, V, max_len=10)
+    ti[:, 0], tw[:, 0] = rng.integers(0, V, size=B), 1.0
+    module = sys.modules["gpusparse.search"]
+    workspace = module._workspace
+
+    def small(index, nbytes, stream_key=0, plan=None):
+        if plan[0] == "scorer":
+            raise torch.cuda.OutOfMemoryError("no room")
+        return workspace(index, nbytes, stream_key, plan)
+
+    monkeypatch.setattr(module, "_workspace", small)
+    st = {}
+    check(ix, ref_of(csr), ti, tw, k, "no room")
+    gs.search(ix, (ti, tw), k, path="fused", timing=st)
+    assert st["retried_rows"] > B // 2 and st["dense_rows"] >= st["retried_rows"]
 
 
 def test_block_copy_threads(device, monkeypatch):

@@ -57,6 +57,20 @@ def test_compaction_spans(device, L):
             assert np.array_equal(i.cpu().numpy(), oi) and np.array_equal(v.cpu().numpy(), ov)
 
 
+@pytest.mark.parametrize("L", [300, 4097, 9000])
+def test_compaction_of_nan(device, L):
+    """NaN scores reach no threshold: they are not among the candidates."""
+    rng = np.random.default_rng(L)
+    x = rng.normal(size=(3, L)).astype(np.float32)
+    x[:, ::3] = np.nan
+    x[1, 1::3] = np.copysign(np.float32(np.nan), np.float32(-1))
+    x[2] = np.nan
+    tau = np.array([0.0, -np.inf, -np.inf], np.float32)
+    v, i = gs.compacted_topk(torch.from_numpy(x).to(device), torch.from_numpy(tau).to(device), 250)
+    ov, oi = O.compacted_topk(x, tau, 250)
+    assert np.array_equal(i.cpu().numpy(), oi) and np.array_equal(v.cpu().numpy(), ov)
+
+
 @pytest.mark.parametrize("n_docs", [1, 255, 256, 257, 4095, 4097, 20001])
 @pytest.mark.parametrize("kind", ["f32", "f16", "u8", "repeats", "negative", "few"])
 def test_dense_rows(device, kind, n_docs):
