@@ -414,3 +414,30 @@ def test_block_streams(device):
         for p, (es, _, ei) in zip(pending, want):
             s, i = p.result()
             assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(s.cpu().numpy(), es)
+
+
+@pytest.mark.parametrize("vocab", [57_345, 65_663, 65_664])
+def test_block_vocabulary(device, vocab):
+    """The most tail lists the copy's 16-bit ranks hold, all of them non-empty, and one more,
+    which the block search leaves to the hybrid one."""
+    rng = np.random.default_rng(vocab)
+    n, B = 1500, 512
+    per = -(-vocab // n)
+    rows = [np.unique(np.concatenate([np.arange(d * per, min((d + 1) * per, vocab)),
+                                      rng.integers(0, 400, size=20), rng.integers(0, vocab, size=20)]))
+            for d in range(n)]
+    indptr = np.concatenate([[0], np.cumsum([r.size for r in rows])]).astype(np.int64)
+    idx = np.concatenate(rows).astype(np.int32)
+    csr = gs.CSR(indptr, idx, rng.lognormal(-0.5, 0.8, size=idx.size).astype(np.float32), (n, vocab))
+    ix, ref = gs.build_from_csr(csr, device), ref_of(csr)
+    ti, tw = random_queries(rng, B, vocab, max_len=30)
+    ti[:, ::3] = rng.integers(vocab - 300, vocab, size=ti[:, ::3].shape)
+    tw[:, ::3] = 1.0
+    if vocab == 65_664:
+        assert not gs.search_plan(ix, B, ti.shape[1], 20)["blocks"]
+        s, i = gs.search(ix, (ti, tw), 20, path="fused")
+        es, _, ei = O.c_search(ref, ti, tw, 20, threads=8)
+        assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(s.cpu().numpy(), es)
+        return
+    assert ensure_blocks(ix).n_tail == vocab - H
+    check(ix, ref, ti, tw, 20, f"vocab={vocab}")
