@@ -184,7 +184,7 @@ struct BlkQueries {
     int32_t *shift;  // [slots] r
     int32_t *kq;     // [slots] 128 sum a_h (255 levels)
     double *ct;      // [slots] Ct; 0: no entries (padding, or a row for the dense path)
-    uint2 *tab;      // [chunks][n_tail + 1] entries of each tail term: [x, y); the last one empty
+    uint2 *tab;      // [chunks][n_tail] entries of each tail term: [x, y)
     uint32_t *ent;   // [chunks][ent_ld] qi << 12 | 8 times the query's place in the chunk
     int64_t ent_ld;
     uint32_t *total;  // [chunks] entries handed out
@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(256) k_blk_prep(const BlkQueries a) {
         a.cnt[q] = !ok && M > 0.0 && M < inf ? kBlkPast : 0;
     }
     if (!ok) return;
-    uint2 *tab = a.tab + (int64_t)(q / a.Q) * (a.n_tail + 1);
+    uint2 *tab = a.tab + (int64_t)(q / a.Q) * a.n_tail;
     for (int j = lane; j < a.T; j += 64) {
         const int32_t t = qrow[j];
         if ((uint32_t)t >= (uint32_t)a.V) continue;
@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(1024) k_blk_ranges(uint2 *__restrict__ tab, in
                                                      uint32_t *__restrict__ total, uint64_t *__restrict__ live) {
     __shared__ uint32_t s_wave[16], s_base;
     const int x = blockIdx.x * 1024 + threadIdx.x;
-    uint2 *t = tab + (int64_t)blockIdx.y * (n_tail + 1);
+    uint2 *t = tab + (int64_t)blockIdx.y * n_tail;
     const int wave = threadIdx.x >> 6;
     const uint32_t c = x < n_tail ? t[x].y : 0u;
     const uint32_t inc = gs_wave_incl_scan(c);
@@ -365,7 +365,7 @@ __global__ void __launch_bounds__(256) k_blk_entries(const BlkQueries a) {
         if (rk < kBlkHeavy || !(ct > 0.0)) continue;
         const int c = q / a.Q;
         const int qi = (int)rint((double)a.qw[i] * ct * 1024.0 * (double)a.max_abs[t] / 511.0);  // |qi| < 2^17
-        const uint32_t at = atomicAdd(&a.tab[(int64_t)c * (a.n_tail + 1) + rk - kBlkHeavy].y, 1u);
+        const uint32_t at = atomicAdd(&a.tab[(int64_t)c * a.n_tail + rk - kBlkHeavy].y, 1u);
         a.ent[(int64_t)c * a.ent_ld + at] = ((uint32_t)qi << 12) | (uint32_t)(q - c * a.Q) * 8u;
     }
 }
@@ -484,7 +484,7 @@ __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
     if (lin >= a.sets * a.chunks) return;
     const int chunk = lin % a.chunks;
     const int q0 = chunk * a.Q;  // first slot of the chunk
-    const uint2 *tab = a.tab + (int64_t)chunk * (a.n_tail + 1);
+    const uint2 *tab = a.tab + (int64_t)chunk * a.n_tail;
     const uint32_t *ent = a.ent + (int64_t)chunk * a.ent_ld;
     const int nct = a.Q >> 4;
     const int last = a.place0 + a.n_places;
