@@ -690,12 +690,14 @@ def main():
         t0 = time.perf_counter()
         tile, hyb = scorer_choice(ix, a.tile_log2 or None, want_hybrid)
         sx = search_index(ix, hyb)
-        if a.named or block_copy(sx, a.batch or cfg.queries.n_rows, hyb, True) is None:
+        width = int(np.diff(queries.indptr).max())
+        if a.named or block_copy(sx, a.batch or cfg.queries.n_rows, width, min(a.k or cfg.k, docs.shape[0]), hyb,
+                                 True) is None:
             ensure_search_state(sx, tile, hybrid=hyb)
         torch.cuda.synchronize()
         return ix, ev, t_build, time.perf_counter() - t0, tile, hyb
 
-    a.named = bool(a.tile_log2 or a.scorer != "auto" or a.unroll or a.waves or a.tiles_per_wg or a.sample_tiles)
+    a.named = bool(a.tile_log2 or a.scorer != "auto" or a.unroll or a.tiles_per_wg or a.sample_tiles)
     want_hybrid = {"auto": None, "hybrid": True, "lds": False}[a.scorer]
     index, build_ev, t_build, t_state, a.tile_log2, hyb = build(docs)
     log(f"index built in {t_build:.2f}s (incl. H2D of the CSR); first-search state (tile bounds, packed copy, "

@@ -264,20 +264,43 @@ def dense_preferred(index, B: int, k: int, tile_log2: int, hybrid: bool, dense_b
 
 BLOCK_MIN_QUERIES = 256    # fewest queries of a batch that takes the block search,
 BLOCK_MIN_PAIRS = 280 << 20  # and its fewest (query, doc) pairs
+BLOCK_NARROW_T = 128   # batches up to this wide have no further condition, those
+BLOCK_MAX_T = 256      # up to this one need more queries or docs for many results
+BLOCK_WIDE_K = 1120    # (blocks_preferred)
 
 
-def block_copy(index, B: int, hybrid: bool, default_scorer: bool):
+def blocks_preferred(B: int, T: int, k: int, n_docs: int) -> bool:
+    """Whether the block search is the faster one, against the hybrid search, for a batch
+    of B queries up to T terms wide and k results on n_docs docs.
+
+    It reads every posting of the collection once per 512 queries, whatever they hold,
+    and scores a query at little more than its products; the hybrid search writes and
+    reads a sum per (query, doc).  So it needs some 250 queries, and enough pairs for its
+    launches.  Blocks against hybrid, us per batch of queries of about 30 terms at k =
+    1000: 512 queries on 300K docs 819 / 815, on 600K 1027 / 1206, on 1M 1247 / 1436, on
+    8.8M 5054 / 7691; 1024 on 1M 2119 / 2689; 300 on 1M 971 / 985; 256 on 3M 1701 / 1712,
+    on 8.8M 3823 / 4026; 200 on 3M 1477 / 1350; 64 on 3M 1094 / 645.
+
+    Its margin grows with the query's terms (int16 sums, levels of each list's largest
+    weight), and with it the docs rescored around the k-th: about 1 us per query more than
+    the hybrid search at 80 to 150 terms and k = 1000, against a gain of 0.2 us per 100
+    queries beyond 240 and million docs.  80 terms (batches 256 wide), k = 1000: 512
+    queries on 600K docs 1560 / 1531, on 1M 1877 / 1900, on 3M 3375 / 4166; 300 on 1M
+    1482 / 1269; 256 on 3M 2472 / 2258; 1024 on 1M 3186 / 3540; at k = 10 300 on 1M 798 /
+    817.  150 terms: 512 on 1M 2862 / 2527, on 3M 5039 / 5583; 300 on 1M 2098 / 1631.
+    At 310 terms (600 wide) 512 queries on 1M docs take 3714 / 2775 at k = 10 and 8831 /
+    4501 at k = 1000, on 3M 7453 / 7443 and 14004 / 9700."""
+    pairs = B * n_docs
+    if B < BLOCK_MIN_QUERIES or pairs < BLOCK_MIN_PAIRS or T > BLOCK_MAX_T:
+        return False
+    return T <= BLOCK_NARROW_T or pairs - (BLOCK_MIN_QUERIES - 16) * n_docs >= BLOCK_MIN_PAIRS * k // BLOCK_WIDE_K
+
+
+def block_copy(index, B: int, T: int, k: int, hybrid: bool, default_scorer: bool):
     """The index's block copy when a fused search of B queries runs on it (built on
-    first use), else None: batches that would take the hybrid search and name neither
-    scorer nor launch shape, of at least BLOCK_MIN_QUERIES and BLOCK_MIN_PAIRS.
-    The block search reads every posting of the collection once per 512 queries,
-    whatever they hold, and scores a query at little more than its products; the
-    hybrid search writes and reads a sum per (query, doc).  Blocks against hybrid,
-    us per batch at k = 1000: 512 queries on 300K docs 819 / 815, on 1M 1235 / 1416,
-    on 8.8M 4980 / 7485; 1024 on 1M 2121 / 2690; 256 on 1M 838 / 838, on 3M 1632 /
-    1715; 200 on 3M 1477 / 1350; 64 on 3M 1094 / 645."""
-    if not (hybrid and default_scorer and B >= BLOCK_MIN_QUERIES and
-            B * int(index.num_docs) >= BLOCK_MIN_PAIRS and blocks_eligible(index)):
+    first use), else None: batches that would take the hybrid search, name neither
+    scorer nor launch shape, and that it is the faster one for."""
+    if not (hybrid and default_scorer and blocks_preferred(B, T, k, int(index.num_docs)) and blocks_eligible(index)):
         return None
     return ensure_blocks(index)
 
@@ -432,7 +455,7 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
     ref = _lib.C.byref
     opts = _opts(sample_tiles, cand_cap, unroll, waves, tiles_per_wg, batch_order, hyb)
     need = _lib.C.c_size_t()
-    blocks = block_copy(index, B, hyb, default_scorer)
+    blocks = block_copy(index, B, T, kk, hyb, default_scorer)
     if blocks is not None:
         gidx, bcopy = gs_blocks_index(index), blocks.struct()
         _lib.check(L.gs_search_blocks_workspace(ref(gidx), ref(bcopy), B, T, kk, ref(opts), ref(need)),
@@ -547,7 +570,7 @@ def search_plan(index, B: int, T: int, k: int, *, tile_log2: int | None = None, 
     default_scorer = _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch_order)
     tile_log2, hyb = scorer_choice(index, tile_log2, hybrid, T)
     index = search_index(index, hyb)
-    if block_copy(index, int(B), hyb, default_scorer) is not None:
+    if block_copy(index, int(B), int(T), min(int(k), int(index.num_docs)), hyb, default_scorer) is not None:
         return {"tile_log2": tile_log2, "seed_tiles": None, "group_size": None, "unroll": None, "tiles_per_wg": None,
                 "packed": None, "hybrid": hyb, "cand_cap": None, "blocks": True}
     gidx = gs_index_struct(index, tile_log2, hyb)
@@ -575,7 +598,7 @@ def search_counts(index, B: int, T: int, k: int, *, tile_log2: int | None = None
         raise ValueError("no fused search has run on this index")
     dev = _device_of(index)
     kk = min(int(k), int(index.num_docs))
-    blocks = block_copy(index, int(B), hyb, default_scorer)
+    blocks = block_copy(index, int(B), int(T), kk, hyb, default_scorer)
     if plan != _plan_key(blocks is not None, B, T, kk, cand_cap, tile_log2, hyb, sample_tiles, unroll, tiles_per_wg,
                          batch_order):
         raise ValueError(f"the last fused search on this index ran with other arguments: {plan}")

@@ -166,3 +166,17 @@ def test_bench_refuses_more_than_one_gpu():
                        text=True, timeout=120, cwd=ROOT)
     assert r.returncode == 2
     assert "measures one GPU" in r.stderr and r.stdout == ""
+
+
+@pytest.mark.parametrize("B,T,k,n_docs,want", [
+    (512, 107, 1000, 8_800_000, True), (1024, 107, 1000, 1_000_000, True), (300, 107, 10, 1_000_000, True),
+    (255, 30, 10, 8_800_000, False), (512, 30, 1000, 500_000, False),
+    # wide batches: many results need more queries or docs
+    (512, 256, 1000, 1_000_000, True), (512, 256, 1000, 600_000, False), (512, 256, 10, 600_000, True),
+    (300, 256, 1000, 1_000_000, False), (300, 129, 10, 1_000_000, True), (300, 128, 1000, 1_000_000, True),
+    (256, 256, 1000, 3_000_000, False), (256, 256, 100, 3_000_000, True), (512, 256, 1000, 3_000_000, True),
+    (512, 257, 10, 8_800_000, False)])
+def test_blocks_preferred(B, T, k, n_docs, want):
+    """The measured sides of the block search's line."""
+    from gpusparse.search import blocks_preferred
+    assert blocks_preferred(B, T, k, n_docs) is want
