@@ -306,6 +306,21 @@ def state_locked(f):
     return locked
 
 
+def state_once(key):
+    """aux()[key] of an index once it is there, else f(index) with that lock held; f
+    publishes the key when what it stands for is complete."""
+    def wrap(f):
+        @functools.wraps(f)
+        def once(index):
+            a = index.aux()
+            if key in a:
+                return a[key]
+            with _state_lock:
+                return f(index)
+        return once
+    return wrap
+
+
 def check_lists(index) -> tuple[int, int]:
     """(non-ascending lists, non-empty lists); caches the per-list duplicate counts."""
     dev = _device_of(index)
@@ -385,7 +400,7 @@ def heavy_terms(index) -> torch.Tensor:
     return out
 
 
-@state_locked
+@state_once("hybrid_ok")
 def hybrid_eligible(index) -> bool:
     """Whether the hybrid search can serve the index: float weights with a packed
     copy (finite weights), and heavy lists that hold each doc at most once.
@@ -500,7 +515,7 @@ class Blocks(NamedTuple):
         return _lib.GsBlockCopy(*(t.data_ptr() for t in self[:5]), self.n_tail, self.levels)
 
 
-@state_locked
+@state_once("blocks_ok")
 def blocks_eligible(index) -> bool:
     """Whether the block search can serve the index: float weights, all finite, the
     128 longest lists holding each doc once, at most 65535 further non-empty lists."""
@@ -521,7 +536,7 @@ def blocks_eligible(index) -> bool:
     return a["blocks_ok"]
 
 
-@state_locked
+@state_once("blocks")
 def ensure_blocks(index) -> Blocks | None:
     """The block copy of an eligible index and the doc-major copy it is made from,
     built once; None when the GPU has no room for them (the search then takes the

@@ -3,12 +3,14 @@
 ``search(index, query_batch, k)`` is the batched retrieval call: scores and doc
 ids of the k best documents per query, ordered by score descending, ties by doc
 id ascending.  ``triton_fused_score`` (src/triton_kernel.py:159-200) keeps the
-reference's name and signature.  Both run the fused pipeline of ``gs_search``
-(for float indexes whose heavy lists hold each doc once, the hybrid search: the
-heavy terms as int8 matrix products, the others added in LDS score tiles; else
-every term added in LDS) and finish the rare rows it flags with the dense path
-(``gs_search_dense``), or run the dense path directly when the full
-``[B, num_docs]`` score rows are small.
+reference's name and signature.  Both run a fused pipeline and finish the rare
+rows it flags with the dense path (``gs_search_dense``), or run the dense path
+directly when the full ``[B, num_docs]`` score rows are small.  The fused pipeline
+of an index whose heavy lists hold each doc once is the block search
+(``gs_search_blocks``) for large batches (``blocks_preferred``) and the hybrid search
+of ``gs_search`` for the others: both score the heavy terms as int8 matrix products
+and add the other terms in LDS.  Else it is ``gs_search`` with every term added in
+LDS.  uint8 indexes run on a float16 copy of their weights where that is exact.
 
 Float indexes return float32 scores equal to the fp64 scatter-add rounded to
 float32; uint8 indexes return the exact uint32 sums as int32.
@@ -23,8 +25,7 @@ import torch
 
 from . import _lib
 from .index import (DEFAULT_TILE_LOG2_HYBRID, blocks_eligible, default_tile_log2, ensure_blocks, gs_blocks_index,
-                    gs_index_struct, hybrid_eligible, _device_of,
-                    state_locked)
+                    gs_index_struct, hybrid_eligible, state_locked, _device_of)
 
 MAX_K = 8192  # largest k of the fused path and of compacted_topk; search answers larger k densely
 MAX_T = 8192  # widest query batch of the fused path (terms per query); search answers wider ones densely
@@ -221,8 +222,7 @@ def _default_scorer(tile_log2, hybrid, sample_tiles, unroll, tiles_per_wg, batch
 def _plan_key(blocks: bool, B, T, kk, cand_cap, *scorer_args) -> tuple:
     """What lays a fused search's workspace out: the arrays of gs_search_blocks
     follow from the first arguments, those of gs_search from the scorer's too."""
-    return ("blocks" if blocks else "scorer", int(B), int(T), int(kk), int(cand_cap)) + \
-        (() if blocks else tuple(int(x) for x in scorer_args))
+    return ("blocks", B, T, kk, cand_cap) if blocks else ("scorer", B, T, kk, cand_cap, *scorer_args)
 
 
 def _dense_rows(index, gidx, qt, qw, k, rows, out_s, out_i, dense_budget):
@@ -357,7 +357,8 @@ def search(index, query_batch, k: int = 10, *, tile_log2: int | None = None, pat
     tile_log2: doc-tile size of the scorer (default: index.default_tile_log2).
     hybrid: the index's heavy (64 longest) lists as int8 matrix products, the other terms
     as LDS adds (scorer_choice; a uint8 index through its float16 copy); results
-    are the same either way.
+    are the same either way.  A call that names neither of the two nor another
+    launch shape takes the block search where that is faster (blocks_preferred).
     path: "auto" (dense for small batches whose [B, N] rows fit `dense_budget`,
     dense_preferred), "fused" or "dense";
     k above MAX_K (8192) or queries wider than MAX_T (8192 terms) always take the
@@ -502,15 +503,18 @@ def search_async(index, query_batch, k: int = 10, *, tile_log2: int | None = Non
     def finish(status):
         if bad_h is not None and bool(bad_h):
             raise ValueError(_U8_WEIGHTS_MSG)
-        bad = np.nonzero((status != _lib.GS_ROW_DONE) & (status != _lib.GS_ROW_RETRY))[0]
-        retry = np.nonzero(status == _lib.GS_ROW_RETRY)[0]
+        bad = np.flatnonzero(status != _lib.GS_ROW_DONE)
+        if not bad.size and timing is None:
+            return
+        again_rows = status[bad] == _lib.GS_ROW_RETRY
+        bad, retry = bad[~again_rows], bad[again_rows]
         again = {}
         if retry.size:
             # Rows the block search's margin did not settle: a batch of their own, dense
             # or hybrid by the same rule, as its cost per row is a small part of the dense
-            # path's where many are flagged (64 of 512 queries of 300 terms on 1M docs
-            # added 14 ms as dense rows, 1 as a hybrid batch); as dense rows, a few at a
-            # time, where the GPU has no room for that
+            # path's where many are flagged (64 of 512 on 1M docs added 14 ms as dense rows,
+            # 1 as a hybrid batch); as dense rows, a few at a time, where the GPU has no
+            # room for that
             with torch.cuda.stream(stream), _workspace_aside(index, stream.cuda_stream):
                 rows = torch.from_numpy(retry).to(dev)
                 try:
