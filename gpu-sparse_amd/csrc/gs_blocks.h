@@ -173,6 +173,21 @@ __global__ void __launch_bounds__(512)
 
 // ---------------------------------------------------------------------- the batch
 
+// Stride of the order in which the `all` blocks of a collection are taken: coprime to
+// it and about its golden section, so that the blocks of any run of places lie evenly
+// over the whole collection.  Thresholds are fixed while a launch runs, each launch
+// takes as many docs as all before it, and their candidates number about k a launch
+// only if the docs so far are a fair sample of the rest.  In id order they are not
+// where docs lie in topical, date or length order (8.8M docs sorted by the weight of
+// their mid-frequency terms, 512 queries, k = 1000: 11.9 ms in id order, rows past
+// their candidate slots among them, 5.4 in this one; sorted by length 8.4 and 5.4; in
+// no order 5.00 and 5.05).
+inline int32_t blk_stride(int32_t all) {
+    int64_t x = std::max<int64_t>(1, (int64_t)(0.6180339887498949 * all));
+    while (std::gcd(x, (int64_t)all) != 1) ++x;
+    return (int32_t)(x % all);
+}
+
 struct BlkQueries {
     const int32_t *qt;
     const float *qw;
@@ -189,6 +204,10 @@ struct BlkQueries {
     int64_t ent_ld;
     uint32_t *total;  // [chunks] entries handed out
     uint32_t *mfix, *tau, *cnt;
+    const int64_t *row_ptr;  // of the blocks, in the order they are taken in (blk_stride):
+    const int32_t *count;
+    int32_t all, stride;
+    uint4 *place;  // [all] first word (x, y), number of words and block of each place
 };
 
 // One wave per query slot: C, r and Ct (top of the file), the heavy limbs, the
@@ -368,6 +387,14 @@ __global__ void __launch_bounds__(256) k_blk_entries(const BlkQueries a) {
         const uint32_t at = atomicAdd(&a.tab[(int64_t)c * a.n_tail + rk - kBlkHeavy].y, 1u);
         a.ent[(int64_t)c * a.ent_ld + at] = ((uint32_t)qi << 12) | (uint32_t)(q - c * a.Q) * 8u;
     }
+    // where the places' words lie, in their order: neighbouring workgroups of k_blk_score
+    // read neighbouring entries (from the arrays by block each block waited for two
+    // misses of L2, 45 of 5000 us at 8.8M docs, 512 queries)
+    for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < a.all; p += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t b = (uint32_t)((uint64_t)(p * a.stride) % (uint32_t)a.all);
+        const uint64_t s = (uint64_t)a.row_ptr[(int64_t)b * kBlkDocs];
+        a.place[p] = make_uint4((uint32_t)s, (uint32_t)(s >> 32), (uint32_t)a.count[b], b);
+    }
 }
 
 // ---------------------------------------------------------------------- scoring
@@ -375,13 +402,10 @@ __global__ void __launch_bounds__(256) k_blk_entries(const BlkQueries a) {
 struct BlkArgs {
     const int8_t *head;
     const uint32_t *tail;
-    const int32_t *count;
-    const int64_t *row_ptr;
-    int32_t place0, n_places;  // places of this launch in the order the blocks are taken in:
-    int32_t all, stride;       // place p holds block p stride mod all (blk_stride)
+    const uint4 *place;        // BlkQueries::place
+    int32_t place0, n_places;  // places of this launch
     int32_t Q, B, chunks, n_tail;
     int32_t sets;  // workgroups per chunk, each taking every sets-th place
-    int32_t hop;   // sets stride mod all
     const int8_t *alimb;
     const int32_t *shift, *kq;
     const uint2 *tab;
@@ -398,21 +422,6 @@ struct BlkArgs {
     uint32_t *seed;  // SEED: [slots][seed_ld] scores (0 for non-positive ones), by place
     int64_t seed_ld;
 };
-
-// Stride of the order in which the `all` blocks of a collection are taken: coprime to
-// it and about its golden section, so that the blocks of any run of places lie evenly
-// over the whole collection.  Thresholds are fixed while a launch runs, each launch
-// takes as many docs as all before it, and their candidates number about k a launch
-// only if the docs so far are a fair sample of the rest.  In id order they are not
-// where docs lie in topical, date or length order (8.8M docs sorted by the weight of
-// their mid-frequency terms, 512 queries, k = 1000: 11.9 ms in id order, rows past
-// their candidate slots among them, 5.4 in this one; sorted by length 8.4 and 5.4; in
-// no order 5.00 and 5.05).
-inline int32_t blk_stride(int32_t all) {
-    int64_t x = std::max<int64_t>(1, (int64_t)(0.6180339887498949 * all));
-    while (std::gcd(x, (int64_t)all) != 1) ++x;
-    return (int32_t)(x % all);
-}
 
 // Workgroup barrier that orders LDS accesses only: loads from global memory stay in
 // flight across it (__syncthreads waits for them).
@@ -558,14 +567,15 @@ __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
         }
     };
     int place = a.place0 + lin / a.chunks;
-    int blk = (int)((uint64_t)((int64_t)place * a.stride) % (uint32_t)a.all);
-    const uint32_t *words = a.tail + a.row_ptr[(int64_t)blk * kBlkDocs];
-    int n = a.count[blk];
+    auto first_word = [&](const uint4 &p) { return a.tail + (int64_t)((uint64_t)p.y << 32 | p.x); };
+    uint4 here = a.place[place];
+    const uint32_t *words = first_word(here);
+    int n = (int)here.z;
     uint32_t wd[kBlkGroups];
     if (n > 0) load_words(words, n, wave * 64, wd);
 
     for (; place < last; place += a.sets) {
-        const int64_t doc0 = (int64_t)blk * kBlkDocs;
+        const int64_t doc0 = (int64_t)here.w * kBlkDocs;
         gs_v4i av[RT][KB];
         auto load_head = [&]() {
             const int8_t *hp = a.head + doc0 * kBlkHeavy + lane * 16;
@@ -626,10 +636,10 @@ __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
         }
         gs_v4i bl[KB], bh[KB];
         load_limbs(min(wave, nct - 1), bl, bh);
-        if ((blk += a.hop) >= a.all) blk -= a.all;
         if (place + a.sets < last) {
-            words = a.tail + a.row_ptr[(int64_t)blk * kBlkDocs];
-            n = a.count[blk];
+            here = a.place[place + a.sets];
+            words = first_word(here);
+            n = (int)here.z;
             if (n > 0) load_words(words, n, wave * 64, wd);
         }
         blk_barrier();

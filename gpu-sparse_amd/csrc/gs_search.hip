@@ -2718,6 +2718,7 @@ struct BlkPlan {
     uint2 *tab;
     uint64_t *live;
     uint32_t *total, *ent, *seed, *out_q, *out_doc, *out_key, *out_n;
+    uint4 *place;
     int64_t cleared;  // 32-bit words from tab on that each search clears (tab, total)
     int32_t lists;    // scoring workgroups, all chunks
 };
@@ -2765,6 +2766,7 @@ BlkPlan plan_blocks(const gs_index *ix, const gs_block_copy *bk, int32_t B, int3
     p.out_key = ar.take<uint32_t>((size_t)p.lists * kBlkList);
     p.out_n = ar.take<uint32_t>((size_t)p.lists);
     p.live = ar.take<uint64_t>((size_t)p.chunks * blk_live_words(bk->n_tail));
+    p.place = ar.take<uint4>((size_t)((ix->n_docs + kBlkDocs - 1) / kBlkDocs));
     p.ent = ar.take<uint32_t>((size_t)(p.chunks * p.ent_ld));
     p.cand_doc = ar.take<uint32_t>((size_t)B * p.cap);
     p.cand_key = ar.take<uint32_t>((size_t)B * p.cap);
@@ -2835,12 +2837,18 @@ int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_
     bq.mfix = p.mfix;
     bq.tau = p.tau;
     bq.cnt = p.cnt;
+    const int32_t all = (int32_t)((ix->n_docs + kBlkDocs - 1) / kBlkDocs);
+    bq.row_ptr = ix->fwd_ptr_d;
+    bq.count = bk->count_d;
+    bq.all = all;
+    bq.stride = blk_stride(all);
+    bq.place = p.place;
     k_blk_prep<<<gs_blocks((int64_t)p.slots * 64, 256), 256, 0, s>>>(bq);
     GS_CHECK_LAUNCH();
     k_blk_ranges<<<dim3(gs_blocks(bk->n_tail, 1024), (unsigned)p.chunks), 1024, 0, s>>>(p.tab, bk->n_tail, p.total,
                                                                                            p.live);
     GS_CHECK_LAUNCH();
-    k_blk_entries<<<gs_blocks((int64_t)B * T, 256, 4096), 256, 0, s>>>(bq);
+    k_blk_entries<<<gs_blocks(std::max<int64_t>((int64_t)B * T, all), 256, 4096), 256, 0, s>>>(bq);
     GS_CHECK_LAUNCH();
     if ((rc = phase(1))) return rc;
     if ((rc = phase(2))) return rc;
@@ -2854,8 +2862,7 @@ int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_
     BlkArgs a{};
     a.head = bk->head_d;
     a.tail = bk->tail_d;
-    a.count = bk->count_d;
-    a.row_ptr = ix->fwd_ptr_d;
+    a.place = p.place;
     a.Q = p.Q;
     a.B = B;
     a.chunks = p.chunks;
@@ -2881,14 +2888,10 @@ int search_blocks_impl(const gs_index *ix, const gs_block_copy *bk, const int32_
     a.collect = blk_collect(p.Q, bk->n_tail);
     a.seed = p.seed;
     a.seed_ld = p.seed_docs;
-    const int32_t all = (int32_t)((ix->n_docs + kBlkDocs - 1) / kBlkDocs);
-    a.all = all;
-    a.stride = blk_stride(all);
     auto run = [&](bool seed, int32_t p0, int32_t p1) -> int {
         a.place0 = p0;
         a.n_places = p1 - p0;
         a.sets = std::min(a.n_places, p.lists / p.chunks);
-        a.hop = (int32_t)((int64_t)a.sets * a.stride % all);
         const unsigned grid = (unsigned)((a.sets * p.chunks + 7) / 8 * 8);
         const size_t lds = blk_lds_fixed(p.Q, bk->n_tail) + (size_t)a.collect * 12;
         if (seed) k_blk_score<true><<<grid, kBlkThreads, lds, s>>>(a);
