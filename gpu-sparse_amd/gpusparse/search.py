@@ -264,9 +264,11 @@ def dense_preferred(index, B: int, k: int, tile_log2: int, hybrid: bool, dense_b
 
 BLOCK_MIN_QUERIES = 256    # fewest queries of a batch that takes the block search,
 BLOCK_MIN_PAIRS = 280 << 20  # and its fewest (query, doc) pairs
-BLOCK_NARROW_T = 128   # batches up to this wide have no further condition, those
-BLOCK_MAX_T = 256      # up to this one need more queries or docs for many results
-BLOCK_WIDE_K = 1120    # (blocks_preferred)
+BLOCK_NARROW_T = 128   # batches up to this wide have no further condition; wider ones
+BLOCK_WIDE_T = 256     # need more queries or docs for many results, beyond this width
+BLOCK_WIDE_K = 1120    # for k of this (to it) ...
+BLOCK_WIDEST_K = 4     # ... and of this (beyond it) BLOCK_MIN_PAIRS past 240 queries
+BLOCK_ANY_PAIRS = 1 << 34  # pairs from which any batch takes it: the hybrid search's sums, 24 GiB
 
 
 def blocks_preferred(B: int, T: int, k: int, n_docs: int) -> bool:
@@ -288,12 +290,16 @@ def blocks_preferred(B: int, T: int, k: int, n_docs: int) -> bool:
     queries on 600K docs 1560 / 1531, on 1M 1877 / 1900, on 3M 3375 / 4166; 300 on 1M
     1482 / 1269; 256 on 3M 2472 / 2258; 1024 on 1M 3186 / 3540; at k = 10 300 on 1M 798 /
     817.  150 terms: 512 on 1M 2862 / 2527, on 3M 5039 / 5583; 300 on 1M 2098 / 1631.
-    At 310 terms (600 wide) 512 queries on 1M docs take 3714 / 2775 at k = 10 and 8831 /
-    4501 at k = 1000, on 3M 7453 / 7443 and 14004 / 9700."""
+    At 310 terms (600 wide) and k = 10 512 queries on 1M docs take 3714 / 2775, on 3M 7453 /
+    7443, on 8.8M 17223 / 21610, 1024 on 1M 5005 / 5296; at k = 100 512 on 3M 10661 /
+    7778; at k = 1000 512 on 3M 14004 / 9700, on 8.8M 29826 / 24245."""
     pairs = B * n_docs
-    if B < BLOCK_MIN_QUERIES or pairs < BLOCK_MIN_PAIRS or T > BLOCK_MAX_T:
+    if B < BLOCK_MIN_QUERIES or pairs < BLOCK_MIN_PAIRS:
         return False
-    return T <= BLOCK_NARROW_T or pairs - (BLOCK_MIN_QUERIES - 16) * n_docs >= BLOCK_MIN_PAIRS * k // BLOCK_WIDE_K
+    if T <= BLOCK_NARROW_T or pairs >= BLOCK_ANY_PAIRS:
+        return True
+    past = pairs - (BLOCK_MIN_QUERIES - 16) * n_docs
+    return past >= BLOCK_MIN_PAIRS * k // (BLOCK_WIDE_K if T <= BLOCK_WIDE_T else BLOCK_WIDEST_K)
 
 
 def block_copy(index, B: int, T: int, k: int, hybrid: bool, default_scorer: bool):

@@ -175,7 +175,10 @@ def test_bench_refuses_more_than_one_gpu():
     (512, 256, 1000, 1_000_000, True), (512, 256, 1000, 600_000, False), (512, 256, 10, 600_000, True),
     (300, 256, 1000, 1_000_000, False), (300, 129, 10, 1_000_000, True), (300, 128, 1000, 1_000_000, True),
     (256, 256, 1000, 3_000_000, False), (256, 256, 100, 3_000_000, True), (512, 256, 1000, 3_000_000, True),
-    (512, 257, 10, 8_800_000, False)])
+    (512, 600, 10, 1_000_000, False), (1024, 600, 10, 1_000_000, True), (512, 257, 10, 8_800_000, True),
+    (512, 600, 100, 3_000_000, False), (512, 257, 1000, 8_800_000, False),
+    # the hybrid search's sums would take 24 GiB
+    (512, 600, 1000, 33_000_000, False), (512, 600, 1000, 34_000_000, True)])
 def test_blocks_preferred(B, T, k, n_docs, want):
     """The measured sides of the block search's line."""
     from gpusparse.search import blocks_preferred
