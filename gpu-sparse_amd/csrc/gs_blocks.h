@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(512)
 // where docs lie in topical, date or length order (8.8M docs sorted by the weight of
 // their mid-frequency terms, 512 queries, k = 1000: 11.9 ms in id order, rows past
 // their candidate slots among them, 5.4 in this one; sorted by length 8.4 and 5.4; in
-// no order 5.00 and 5.05).
+// no order 4.99 and 5.01).
 inline int32_t blk_stride(int32_t all) {
     int64_t x = std::max<int64_t>(1, (int64_t)(0.6180339887498949 * all));
     while (std::gcd(x, (int64_t)all) != 1) ++x;
@@ -451,8 +451,7 @@ static_assert(blk_lds_fixed(kBlkMaxQ, 65535) + kBlkMinCand * 12 <= kBlkLds,
 //     four per 16-byte load, one ds_add_u32 each into the tile, whose words hold two
 //     docs: a negative sum borrows from the upper one, which the decoding undoes (both
 //     sums fit 16 bits).  The look-ups of the other postings' lanes point past their
-//     buffers and go nowhere: the vector cache takes about one line per clock, which
-//     bounds this part.
+//     buffers and go nowhere: the vector cache takes about one line per clock.
 //  2. products: wave w takes 16-query columns w, w + 8, ...: its C operands are the
 //     tile's sums (cleared as they are read), A the block's head rows (held in
 //     registers, loaded under the tail), B the queries' limbs, loaded a column ahead.
@@ -465,13 +464,14 @@ static_assert(blk_lds_fixed(kBlkMaxQ, 65535) + kBlkMinCand * 12 <= kBlkLds,
 // The tile's 8-byte pieces (4 docs of a query) are XOR-swizzled by the query, so
 // that a wave's C reads (16 queries x 4 pieces) spread over the banks.
 // SEED: the scores themselves go to `seed`, for the first threshold.
-// What bounds it: a block's chain of loads (words, look-ups, entries, head rows)
-// against 16 waves per CU, and the rare path's instructions.  8.8M docs, 512
-// queries, k = 1000: 4.6 ms for all launches, where the hybrid search's products
-// and scorer took 1.7 + 5.4; of 2.6 ms at 4.4M docs the products are 0.7, the tail
-// about 1.2, emission the rest.  (256 heavy terms: 64 more registers of head rows, so
-// half the waves, 3.8 ms at 4.4M.  At 128 they cost 204 tail adds per doc instead of
-// 91, and win.)
+// What bounds it: by the counters no unit alone.  8.8M docs, 512 queries, k = 1000:
+// 4.4 ms for all launches, where the hybrid search's products and scorer took 1.7 +
+// 5.4, with the vector ALU issuing 58% of the time, the vector cache at 0.50 lines per
+// clock and CU, LDS 18%, MFMA 11%, HBM at a tenth; 14.5 of 16 waves per CU are there,
+// and wait half of their time for a block's chain of loads (words, look-ups, entries,
+// head rows) and its barriers.  Emission is about 12% (k = 10: 0.6 ms less).  (256
+// heavy terms: 64 more registers of head rows, so half the waves, 3.8 ms at 4.4M docs
+// against 2.6.  At 128 they cost 204 tail adds per doc instead of 91, and win.)
 template <bool SEED>
 __global__ void __launch_bounds__(kBlkThreads, 4) k_blk_score(const BlkArgs a) {
     constexpr int NW = kBlkThreads / 64;

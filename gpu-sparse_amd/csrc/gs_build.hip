@@ -115,7 +115,7 @@ __global__ void k_term_count_global(const int32_t *__restrict__ idx, int64_t nnz
 // delta = offsets - exclusive scan(lengths).  Single block of 1024 threads: each of
 // its 16 waves sums its run of terms, then scans it 64 terms at a time from the
 // runs before, with two workgroup barriers in all (two scans with three barriers
-// each per 1024 terms took 66 us at V = 30522; now 50).
+// each per 1024 terms took 66 us at V = 30522; now 45 to 51 for its two launches).
 __global__ void __launch_bounds__(1024) k_term_scan(const int32_t *lengths, int32_t V, int32_t *padded,
                                                     int64_t *offsets, int64_t *delta, int64_t *info,
                                                     const unsigned long long *n_bad) {

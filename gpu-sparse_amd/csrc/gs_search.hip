@@ -298,10 +298,10 @@ __device__ __forceinline__ uint32_t dense_bin(double v, float scale) {
 // ds_add_f64 sustains 0.26 lane-adds per clock and CU where a read and a write of
 // 8 bytes sustain several.  Lists with repeated docs take the atomic.
 // What bounds it is latency at one query (the chain bounds -> postings -> adds) and
-// the instructions per (term, 256 docs) at many: about 40 us plus 20 to 27 us per
-// million (query, doc) pairs.  Scores of one query on 100K / 1M docs 425 -> 37 and
-// 515 -> 73 us, of 256 queries on 100K docs 1610 -> ~600, against 16384-doc slices
-// of one wave per CU.  (Fewer workgroups per row, so that a batch of rows fills the
+// the instructions per (term, 256 docs) at many, 24 us per million (query, doc)
+// pairs.  One query on 100K docs 19 us (k = 10, the whole call 34), on 1M 43 us (k =
+// 100, fp16; 64), 256 queries on 100K docs 607, where 16384-doc slices of one wave per
+// CU took 425, 515 and 1610.  (Fewer workgroups per row, so that a batch of rows fills the
 // chip once, left it to the longest query: 64 queries on 100K docs 184 -> 288 us.)
 template <int WT>
 __global__ void __launch_bounds__(64 * kDenseWaves, 4) k_score_dense(const DenseArgs a) {

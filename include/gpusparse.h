@@ -281,8 +281,9 @@ int gs_search(const gs_index *index, const int32_t *q_terms_d, const void *q_wei
 
 /* ------------------------------------------------------------ block search
  * No counterpart in the reference: gs_search's answers from a doc-block-major
- * copy of a float index, for batches of some dozens of queries or more.  Blocks of
- * GS_BLOCK_DOCS docs; the copy is made from the doc-major copy (gs_forward_fill):
+ * copy of a float index.  It is the faster one from about 250 queries on (300 on 1M docs,
+ * 240 on 8.8M): below, reading every posting costs more than the sums it saves.  Blocks
+ * of GS_BLOCK_DOCS docs; the copy is made from the doc-major copy (gs_forward_fill):
  *   rank_d   int32 [vocab]: the lists by length, longest first: 0 .. GS_BLOCK_HEAVY - 1
  *            the heavy terms, GS_BLOCK_HEAVY + x the tail terms x = 0 .. n_tail - 1, -1
  *            for empty lists (n_tail <= 65535); max_abs_d as in gs_index
